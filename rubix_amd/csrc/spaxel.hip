@@ -9,21 +9,26 @@
 //   keys are bucketed into B = n_keys + 1 buckets (the last one collects ids
 //   outside [0, n_keys)); the input is cut into tiles, each tile owned by one
 //   wavefront that walks it in order, 64 stars per round.
-//   1. count  : per (bucket, tile) counts.  Lanes with equal keys in a round
-//               are found with one ballot per key bit; the lowest lane adds
-//               the group size.  Only the tile's own wavefront touches a
-//               (bucket, tile) counter, so the result is deterministic.
+//   1. rank   : lanes with equal keys in a round are found with one ballot per
+//               key bit; the lowest lane adds the group size to the tile's
+//               (bucket, tile) counter and gets the count so far, so every
+//               star's rank among the tile's stars of its key is known (and
+//               stored) after one walk.  Only the tile's own wavefront touches
+//               a counter, so the result is deterministic.
 //   2. scan   : exclusive scan over the bucket-major (bucket, tile) table
 //               gives each tile its base position inside each bucket.
-//   3. scatter: the same walk; position = base + rank inside the round's
-//               equal-key group, so stars keep their input order (stable).
-//   The (bucket, tile) table of 4096-star tiles is kept to 2^24 entries.  Key
-//   counts past that (a batch of many galaxies: 310 000 keys over 31.8 M
-//   stars) sort in LSD radix passes over D-bit digits of the bucket index,
-//   each pass the same stable count + scan + scatter over 2^D buckets, the
-//   scatter carrying each star's input index and bucket along; stable
-//   passes give the same order as the one-pass sort.  Bucket offsets then
-//   come from a binary search of the sorted buckets.
+//   3. scatter: thread / star, position = base + rank: stars keep their input
+//               order (stable).
+//   A walk is a chain of rounds of about 1 us each (the counter's round trip),
+//   the table costs about 4 ps an entry (filled, read twice, written once):
+//   plan_tile() takes the tile that balances the two.  The table is kept to
+//   2^24 entries.  Key counts past that with 4096-star tiles (a batch of many
+//   galaxies: 310 000 keys over 31.8 M stars) sort in LSD radix passes over
+//   D-bit digits of the bucket index, each pass the same stable rank + scan +
+//   scatter over 2^D buckets, the scatter carrying each star's input index
+//   and bucket along; stable passes give the same order as the one-pass sort.
+//   Bucket offsets then come from a binary search of the sorted buckets.
+#include <math.h>
 #include <stdarg.h>
 #include <string.h>
 
@@ -131,10 +136,24 @@ __global__ void scan_top_kernel(int32_t* __restrict__ sums, int64_t nblk) {
 }
 
 // Each block: exclusive scan of its kScanBlock elements (thread-contiguous
-// runs of kScanItems) plus the block offset, in place.
-__global__ void scan_down_kernel(int32_t* __restrict__ data, int64_t n,
-                                 const int32_t* __restrict__ block_off) {
+// runs of kScanItems) plus the block offset, in place.  kSums: block_off
+// holds the blocks' own sums and the offset is the sum of the earlier ones
+// (at most kScanSelf of them: a few loads a thread, one launch fewer);
+// otherwise scan_top_kernel has scanned them.
+constexpr int64_t kScanSelf = 4096;
+
+template <bool kSums>
+__global__ void __launch_bounds__(kScanThreads) scan_down_kernel(
+    int32_t* __restrict__ data, int64_t n, const int32_t* __restrict__ block_off) {
   __shared__ int32_t smem[kScanThreads];
+  int32_t off;
+  if (kSums) {
+    int32_t part = 0;
+    for (int b = threadIdx.x; b < int(blockIdx.x); b += kScanThreads) part += block_off[b];
+    block_exclusive_scan<int32_t>(part, smem, &off);
+  } else {
+    off = block_off[blockIdx.x];
+  }
   const int64_t base = int64_t(blockIdx.x) * kScanBlock + int64_t(threadIdx.x) * kScanItems;
   int32_t v[kScanItems];
   int32_t s = 0;
@@ -145,7 +164,7 @@ __global__ void scan_down_kernel(int32_t* __restrict__ data, int64_t n,
     s += v[k];
   }
   int32_t tot;
-  int32_t ex = block_exclusive_scan<int32_t>(s, smem, &tot) + block_off[blockIdx.x];
+  int32_t ex = block_exclusive_scan<int32_t>(s, smem, &tot) + off;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
     int64_t i = base + k;
@@ -170,47 +189,65 @@ struct SortPlan {
 };
 
 constexpr int64_t kTableCap = int64_t(1) << 24;  // (bucket, tile) counters
-constexpr int64_t kSortTile = 4096;              // stars per tile
+constexpr int64_t kSortTile = 4096;              // most stars per tile
+
+// Stars per tile for `buckets` counters a tile: tile / 64 rounds of ~1 us
+// against buckets * n / tile table entries of ~4 ps, least at
+// tile = sqrt(2.56e-4 buckets n), within [64, kSortTile].  Measured at 1 M
+// stars and 2500 keys: rank + scatter + table 182 us at 4096 stars per tile.
+static int64_t plan_tile(int64_t n, int64_t buckets) {
+  const double t = sqrt(2.56e-4 * double(buckets) * double(n));
+  int64_t tile = t >= double(kSortTile) ? kSortTile : (int64_t(t) + 63) / 64 * 64;
+  if (tile < 64) tile = 64;
+  while (tile < kSortTile && buckets * ((n + tile - 1) / tile) > kTableCap) tile += 64;
+  return tile;
+}
 
 static SortPlan make_plan(int64_t n, int32_t n_keys) {
   SortPlan p;
   p.n = n;
   p.n_keys = n_keys;
   p.buckets = n_keys + 1;
-  p.tile = kSortTile;
-  p.ntiles = n > 0 ? (n + p.tile - 1) / p.tile : 1;
   int b = 1;
   while ((int64_t(1) << b) < p.buckets) ++b;
   p.nbits = b;
-  if (int64_t(p.buckets) * p.ntiles <= kTableCap) {
+  const int64_t most = n > 0 ? (n + kSortTile - 1) / kSortTile : 1;  // tiles at the largest tile
+  int64_t buckets = p.buckets;
+  if (int64_t(p.buckets) * most <= kTableCap) {
     p.digit_bits = 0;
     p.passes = 1;
-    p.table = int64_t(p.buckets) * p.ntiles;
   } else {
-    // ntiles <= 2^19 for n < 2^31, so digits of at least 5 bits fit
+    // most <= 2^19 for n < 2^31, so digits of at least 5 bits fit; then the
+    // fewest equal digits of that many passes
     int d = 16;
-    while (d > 1 && (int64_t(1) << d) * p.ntiles > kTableCap) --d;
-    p.digit_bits = d;
+    while (d > 1 && (int64_t(1) << d) * most > kTableCap) --d;
     p.passes = (p.nbits + d - 1) / d;
-    p.table = (int64_t(1) << d) * p.ntiles;
+    p.digit_bits = (p.nbits + p.passes - 1) / p.passes;
+    buckets = int64_t(1) << p.digit_bits;
   }
+  p.tile = plan_tile(n, buckets);
+  p.ntiles = n > 0 ? (n + p.tile - 1) / p.tile : 1;
+  p.table = buckets * p.ntiles;
   p.nblk = (p.table + kScanBlock - 1) / kScanBlock;
   return p;
 }
 
-// Radix passes keep the input index and bucket of every position: three
-// n-element buffers (one index, two buckets) beside the caller's perm.
+// Every star's rank in its tile, and for radix passes the input index and
+// bucket of every position: three n-element buffers (one index, two buckets)
+// beside the caller's perm.
 template <class S>
 static void sort_layout(S& c, const SortPlan& p, int32_t** table, int32_t** blocks,
-                        int32_t** tperm, int32_t** b0, int32_t** b1) {
+                        uint16_t** rank, int32_t** tperm, int32_t** b0, int32_t** b1) {
   auto* t = c.template take<int32_t>(p.table);
   auto* bl = c.template take<int32_t>(p.nblk + 1);
+  auto* rk = c.template take<uint16_t>(p.n > 0 ? p.n : 1);
   const int64_t rn = p.digit_bits ? (p.n > 0 ? p.n : 1) : 0;
   auto* tp = c.template take<int32_t>(rn);
   auto* x0 = c.template take<int32_t>(rn);
   auto* x1 = c.template take<int32_t>(rn);
   if (table) *table = reinterpret_cast<int32_t*>(t);
   if (blocks) *blocks = reinterpret_cast<int32_t*>(bl);
+  if (rank) *rank = reinterpret_cast<uint16_t*>(rk);
   if (tperm) *tperm = reinterpret_cast<int32_t*>(tp);
   if (b0) *b0 = reinterpret_cast<int32_t*>(x0);
   if (b1) *b1 = reinterpret_cast<int32_t*>(x1);
@@ -240,48 +277,60 @@ __device__ inline uint64_t peer_mask(int key, uint64_t active, int nbits) {
   return peers;
 }
 
-// One counting-sort pass.  The sort key of element i is its bucket
-// bucket_of(in[i]), or with mask != 0 the digit (bucket >> shift) & mask.
-// Scatter: perm[pos] = the element's input index (src_perm[i], or i on the
-// first pass), bucket_out[pos] = its bucket, sorted[pos] = its original id
-// (ids[perm[pos]]; in[i] itself on the first pass).
-template <bool kScatter>
-__global__ void __launch_bounds__(64) sort_walk_kernel(
-    const int32_t* __restrict__ in, int64_t n, int32_t n_keys, int64_t tile,
-    int64_t ntiles, int nbits, int shift, int32_t mask, int32_t* __restrict__ table,
-    const int32_t* __restrict__ src_perm, const int32_t* __restrict__ ids,
-    int32_t* __restrict__ perm, int32_t* __restrict__ bucket_out,
-    int32_t* __restrict__ sorted) {
-  // blockDim.x == 64: one wavefront walks one tile in input order.
+// The sort key of element i is its bucket bucket_of(in[i]), or with mask != 0
+// the digit (bucket >> shift) & mask.
+__device__ inline int sort_key(int full, int shift, int32_t mask) {
+  return mask ? ((full >> shift) & mask) : full;
+}
+
+// One wavefront walks one tile in input order: rank[i] = number of earlier
+// stars of the tile with the same key (< tile <= 4096), table[key][tile] = the
+// tile's count of the key.  The next round's keys are loaded ahead of this
+// round's counter round trip.  Bound by that chain: 64 rounds of 4096-star
+// tiles took 54-76 us for any star count from 10 k up, and a second such
+// walk scattered; 10 k stars now take one round.
+__global__ void __launch_bounds__(64) sort_rank_kernel(
+    const int32_t* __restrict__ in, int64_t n, int32_t n_keys, int64_t tile, int64_t ntiles,
+    int nbits, int shift, int32_t mask, int32_t* __restrict__ table, uint16_t* __restrict__ rank) {
   const int lane = threadIdx.x;
   const int64_t t = blockIdx.x;
   const int64_t begin = t * tile;
   const int64_t end = begin + tile < n ? begin + tile : n;
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int32_t next = begin + lane < end ? in[begin + lane] : 0;
   for (int64_t r = begin; r < end; r += 64) {
     const int64_t i = r + lane;
     const bool valid = i < end;
-    const int32_t id = valid ? in[i] : 0;
-    const int full = bucket_of(id, n_keys);
-    const int key = mask ? ((full >> shift) & mask) : full;
+    const int key = sort_key(bucket_of(next, n_keys), shift, mask);
+    next = i + 64 < end ? in[i + 64] : 0;
     const uint64_t active = __ballot(valid);
     const uint64_t peers = peer_mask(key, active, nbits);  // all lanes take part
     const int leader = __ffsll((unsigned long long)peers) - 1;
-    const int cnt = __popcll(peers);
-    const int rank = __popcll(peers & lt_mask);
-    int32_t* slot = table + int64_t(key) * ntiles + t;
     int32_t base = 0;
-    if (valid && lane == leader) base = atomicAdd(slot, cnt);
-    if (kScatter) {
-      base = __shfl(base, leader < 0 ? 0 : leader, 64);
-      if (valid) {
-        const int32_t pos = base + rank;
-        const int32_t src = src_perm ? src_perm[i] : int32_t(i);
-        perm[pos] = src;
-        if (bucket_out) bucket_out[pos] = full;
-        if (sorted) sorted[pos] = src_perm ? ids[src] : id;
-      }
-    }
+    if (valid && lane == leader) base = atomicAdd(table + int64_t(key) * ntiles + t, __popcll(peers));
+    base = __shfl(base, leader < 0 ? 0 : leader, 64);
+    if (valid) rank[i] = uint16_t(base + __popcll(peers & lt_mask));
+  }
+}
+
+// pos = the star's base in the scanned table + its rank: perm[pos] = the
+// element's input index (src_perm[i], or i on the first pass), bucket_out[pos]
+// = its bucket, sorted[pos] = its original id (ids[perm[pos]]; in[i] itself on
+// the first pass).
+__global__ void __launch_bounds__(256) sort_scatter_kernel(
+    const int32_t* __restrict__ in, int64_t n, int32_t n_keys, uint32_t tile, int64_t ntiles,
+    int shift, int32_t mask, const int32_t* __restrict__ table, const uint16_t* __restrict__ rank,
+    const int32_t* __restrict__ src_perm, const int32_t* __restrict__ ids,
+    int32_t* __restrict__ perm, int32_t* __restrict__ bucket_out, int32_t* __restrict__ sorted) {
+  for (int64_t i = gtid(); i < n; i += int64_t(gridDim.x) * blockDim.x) {
+    const int32_t id = in[i];
+    const int full = bucket_of(id, n_keys);
+    const int key = sort_key(full, shift, mask);
+    const int32_t pos = table[int64_t(key) * ntiles + uint32_t(i) / tile] + int32_t(rank[i]);
+    const int32_t src = src_perm ? src_perm[i] : int32_t(i);
+    perm[pos] = src;
+    if (bucket_out) bucket_out[pos] = full;
+    if (sorted) sorted[pos] = src_perm ? ids[src] : id;
   }
 }
 
@@ -315,9 +364,16 @@ static int grid_for(int64_t n, int threads, int64_t cap = 65536) {
 int exclusive_scan_i32(int32_t* data, int64_t n, int32_t* blocks, hipStream_t s) {
   const int64_t nblk = (n + kScanBlock - 1) / kScanBlock;
   if (nblk == 0) return RBX_OK;
-  hipLaunchKernelGGL(scan_reduce_kernel, dim3(nblk), dim3(kScanThreads), 0, s, data, n, blocks);
-  hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(kScanThreads), 0, s, blocks, nblk);
-  hipLaunchKernelGGL(scan_down_kernel, dim3(nblk), dim3(kScanThreads), 0, s, data, n, blocks);
+  if (nblk > 1)
+    hipLaunchKernelGGL(scan_reduce_kernel, dim3(nblk), dim3(kScanThreads), 0, s, data, n, blocks);
+  if (nblk > kScanSelf) {
+    hipLaunchKernelGGL(scan_top_kernel, dim3(1), dim3(kScanThreads), 0, s, blocks, nblk);
+    hipLaunchKernelGGL(scan_down_kernel<false>, dim3(nblk), dim3(kScanThreads), 0, s, data, n,
+                       blocks);
+  } else {
+    hipLaunchKernelGGL(scan_down_kernel<true>, dim3(nblk), dim3(kScanThreads), 0, s, data, n,
+                       blocks);
+  }
   return check_launch("exclusive_scan_i32");
 }
 
@@ -329,7 +385,7 @@ void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s) {
 size_t sort_workspace_size(int64_t n, int32_t n_keys) {
   SortPlan p = make_plan(n, n_keys);
   SizerAdapter a;
-  sort_layout(a, p, nullptr, nullptr, nullptr, nullptr, nullptr);
+  sort_layout(a, p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
   return a.s.used;
 }
 
@@ -341,31 +397,28 @@ size_t sort_workspace_bound(int64_t n, int32_t max_keys) {
   p.table = kTableCap;
   p.nblk = (p.table + kScanBlock - 1) / kScanBlock;
   SizerAdapter a;
-  sort_layout(a, p, nullptr, nullptr, nullptr, nullptr, nullptr);
+  sort_layout(a, p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
   return a.s.used;
 }
 
-// Count + scan of one pass; returns the launch status.
+// Rank, scan and scatter of one pass; returns the launch status.
 static int sort_pass(const SortPlan& p, const int32_t* in, int shift, int32_t mask, int nbits,
-                     int32_t* table, int32_t* blocks, int64_t table_n, const int32_t* src_perm,
+                     int32_t* table, int32_t* blocks, uint16_t* rank, const int32_t* src_perm,
                      const int32_t* ids, int32_t* perm, int32_t* bucket_out, int32_t* sorted,
                      int32_t* offsets, hipStream_t s) {
-  fill_i32(table, table_n, 0, s);
-  if (p.n > 0) {
-    hipLaunchKernelGGL(sort_walk_kernel<false>, dim3(p.ntiles), dim3(64), 0, s, in, p.n,
-                       p.n_keys, p.tile, p.ntiles, nbits, shift, mask, table, nullptr, nullptr,
-                       nullptr, nullptr, nullptr);
-  }
-  int rc = exclusive_scan_i32(table, table_n, blocks, s);
+  fill_i32(table, p.table, 0, s);
+  if (p.n > 0)
+    hipLaunchKernelGGL(sort_rank_kernel, dim3(p.ntiles), dim3(64), 0, s, in, p.n, p.n_keys, p.tile,
+                       p.ntiles, nbits, shift, mask, table, rank);
+  int rc = exclusive_scan_i32(table, p.table, blocks, s);
   if (rc) return rc;
   if (offsets)
     hipLaunchKernelGGL(sort_offsets_kernel, dim3(grid_for(int64_t(p.n_keys) + 1, 256)), dim3(256),
                        0, s, table, p.n_keys, p.ntiles, offsets);
-  if (p.n > 0) {
-    hipLaunchKernelGGL(sort_walk_kernel<true>, dim3(p.ntiles), dim3(64), 0, s, in, p.n, p.n_keys,
-                       p.tile, p.ntiles, nbits, shift, mask, table, src_perm, ids, perm,
-                       bucket_out, sorted);
-  }
+  if (p.n > 0)
+    hipLaunchKernelGGL(sort_scatter_kernel, dim3(grid_for(p.n, 256)), dim3(256), 0, s, in, p.n,
+                       p.n_keys, uint32_t(p.tile), p.ntiles, shift, mask, table, rank, src_perm,
+                       ids, perm, bucket_out, sorted);
   return check_launch("rbx_spaxel_sort");
 }
 
@@ -376,10 +429,11 @@ int spaxel_sort_impl(const int32_t* ids, int64_t n, int32_t n_keys, int32_t* per
   SortPlan p = make_plan(n, n_keys);
   Carver c(ws, ws_bytes);
   int32_t *table = nullptr, *blocks = nullptr, *tperm = nullptr, *b0 = nullptr, *b1 = nullptr;
-  sort_layout(c, p, &table, &blocks, &tperm, &b0, &b1);
+  uint16_t* rank = nullptr;
+  sort_layout(c, p, &table, &blocks, &rank, &tperm, &b0, &b1);
   if (!c.ok) return fail(RBX_EWORKSPACE, "rbx_spaxel_sort: workspace too small");
   if (!p.digit_bits)
-    return sort_pass(p, ids, 0, 0, p.nbits, table, blocks, p.table, nullptr, ids, perm, nullptr,
+    return sort_pass(p, ids, 0, 0, p.nbits, table, blocks, rank, nullptr, ids, perm, nullptr,
                      sorted, offsets, s);
   // LSD radix: pass q sorts by bits [q D, q D + D) of the bucket, stably;
   // the index buffers alternate so that the last pass writes perm
@@ -392,7 +446,7 @@ int spaxel_sort_impl(const int32_t* ids, int64_t n, int32_t n_keys, int32_t* per
     int32_t* pout = ((p.passes - 1 - q) & 1) ? tperm : perm;
     int32_t* bout = bufs[q & 1];
     const int width = last ? p.nbits - q * p.digit_bits : p.digit_bits;
-    int rc = sort_pass(p, in, q * p.digit_bits, mask, width, table, blocks, p.table, src, ids,
+    int rc = sort_pass(p, in, q * p.digit_bits, mask, width, table, blocks, rank, src, ids,
                        pout, bout, last ? sorted : nullptr, nullptr, s);
     if (rc) return rc;
     in = bout;
