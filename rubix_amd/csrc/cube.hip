@@ -711,28 +711,38 @@ __global__ void __launch_bounds__(64) cube_accum_kernel(
   }
 }
 
-// Bins per lane of the fused pass: NB = 4 for targets of up to 4096 bins
-// (8 slabs x 2 wavefronts x 64 lanes x 4), up to 8 for 8192.
+// Strided bins per lane of the fused pass: NB = 4 for targets of up to 4096
+// bins (16 wavefronts x 64 lanes x 4), up to 8 for 8192.
 constexpr int kMaxFusedBins = 8;
 
 // Normalisation and accumulation in one pass for ascending targets: item q
-// is spaxel chunk q, one workgroup of 16 wavefronts, two per lambda slab
-// (wavefront 2b + h takes the bins j0 + 64 NB h + lane + 64 t, t < NB, of
-// slab b; NB = 4 up to 4096 target bins).  The chunk's star states are
-// staged in LDS, 64 at a time.  Per star each wavefront takes its knot
-// window from the locator guesses of its first and last bin, stages the
-// window's shifted knots and spectrum values in its own LDS (no other
-// wavefront reads them) and evaluates P_j on its bins once (the per-bin
-// arithmetic of star_norm_kernel and cube_accum_kernel), then posts four
-// shares of Nn = sum_j P_j dtarget_j; after one barrier (one per two stars,
-// both stars' shares posted first) every wavefront adds the 64 shares in a
-// fixed order, forms sf = nan_to_num(T / Nn) and
-// accumulates P_j sf into its f64 registers.  The shares are
-// double-buffered, so a wavefront may post the next star's share while
-// another still reads this one's.  Each (star, bin) value is computed once
-// instead of twice.  The first wavefront stores sf and Nn for the adjoint.
+// is spaxel chunk q, one workgroup of ceil(n / 64 NB) wavefronts, wavefront w
+// on the bins [64 NB w, 64 NB (w + 1)).  Per star each wavefront takes its knot window from the locator
+// guesses of its first and last bin, stages the window in its own LDS (no
+// other wavefront reads it) and evaluates P_j on its bins once, then posts its
+// share of Nn = sum_j P_j dtarget_j; after one barrier (one per two stars,
+// both stars' shares posted first) every wavefront adds the shares in a fixed
+// order, forms sf = nan_to_num(T / Nn) and accumulates P_j sf into its f64
+// registers.  The shares are double-buffered, so a wavefront may post the
+// next star's share while another still reads this one's.  The first
+// wavefront stores sf and Nn for the adjoint.
+//
+// The bins of a lane:
+// * runs (run_values; knots well sparser than the bins, fused_runs()): kRuns
+//   runs of four consecutive bins.  One locator probe and one exact next-knot
+//   test place a run's first bin in its segment; the others lie in that
+//   segment or the one or two after it, whose left knots, values and slopes
+//   the lane reads once and picks by compares.  The slope
+//   (S_{k+1} - S_k) / (w_{k+1} - w_k) is formed per knot when the window is
+//   staged, so a bin costs no reciprocal.  10 M stars -> 3721 bins, 1000
+//   knots: 41.4 ms strided, 23.5 ms with two runs per lane (39.0 with one:
+//   the per-star work of a wavefront weighs as much as its bins').
+// * strided (strided_values; denser knots, coarse locators): every 64th bin,
+//   each with its own probe, segment reads and reciprocal.  Where a run
+//   crosses three knots or more its reads conflict in LDS: runs took 11.6 ms
+//   against 6.4 ms at 1 M stars -> 3721 bins with 0.8 knots per bin.
 constexpr int kFusedWaves = 2 * kSlabs;
-static_assert(kFusedWaves == 16, "the Nn shares fill one 64-lane wave: 16 waves x 4 rows");
+constexpr int kRunKnots = 240;  // knots of a staged window of runs
 
 // v + the row-of-16 DPP move of v (every lane of the wave active).
 template <int kCtrl>
@@ -749,7 +759,6 @@ __device__ inline float row_sum16(float v) {
   v = plus_dpp<0x124>(v);  // row_ror:4
   return plus_dpp<0x128>(v);  // row_ror:8
 }
-
 // Sum over the 64 lanes in a fixed order, broadcast: the four row sums of
 // row_sum16, added row 0 to row 3.  DPP moves and lane reads only (no LDS
 // round trips).  All 64 lanes must be active.
@@ -761,63 +770,331 @@ __device__ inline float wave_sum_dpp(float v) {
   const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
   return ((r0 + r1) + r2) + r3;
 }
+
+// Sum over the 64 lanes in a fixed order, in lane 63: the four row sums of
+// row_sum16, rows 0 and 1, rows 2 and 3, then the two pairs (DPP row
+// broadcasts; the other lanes hold partial sums).
+__device__ inline float wave_sum_last(float v) {
+  v = row_sum16(v);
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
+}
+
 // Knots of a wavefront's staged window: 80 per bin of a lane (the 64 NB
 // bins of a wavefront span ~64 NB x 1.25 A, ~57 NB knots of a 1.4 A grid,
 // plus the margins); wider windows take the global search.
 template <int NB>
 constexpr int fused_window() { return 80 * NB; }
 
-// Star states staged in LDS per batch: the per-star fields come from LDS
-// (broadcast reads) instead of a global round trip ahead of every star.
-constexpr int kStateBatch = 64;
-
 // A wave-uniform float (the lanes hold the same value) in a scalar register.
 __device__ inline float uniform_f(float v) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
-// Up to 4 bins per lane the kernel holds to 64 VGPRs (8 wavefronts per
-// SIMD); more bins per lane take 128 (4 per SIMD).
-template <bool kDust, int NB>
-__global__ void __launch_bounds__(64 * kFusedWaves)
-__attribute__((amdgpu_waves_per_eu(NB <= 4 ? 8 : 4)))
-cube_fused_kernel(SspView g, rbx_target tg, StarState* __restrict__ state,
-                  const ChunkDesc* __restrict__ desc, const int32_t* __restrict__ n_chunks_ptr,
-                  int slab_bins, int64_t n_items, const float* __restrict__ axav,
-                  double* __restrict__ partial) {
+// The next lane's v (DPP wave shift left by one); lane 63 reads 0.
+__device__ inline float next_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+
+// The lane before's v (DPP wave shift right by one); lane 0 keeps `first`.
+__device__ inline float prev_lane(float v, float first) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138,
+                                                    0xF, 0xF, false));
+}
+
+// P of four ascending bins x whose first lies in the staged segment l or
+// l + 1 (l from the locator guess) and whose bin t lies at most min(t, K)
+// segments after the first: left knots W, values S and slopes D of the K + 1
+// candidate segments are read once, compares pick each bin's.  Returns false
+// (P unset) where a bin lies outside its candidates.
+template <int K>
+__device__ inline bool run_segments(const float (&x)[4], int l, const float* W, const float* S,
+                                    const float* D, float* P) {
+  l += W[l + 1] <= x[0] ? 1 : 0;
+  float w[K + 2], s[K + 1], d[K + 1];
+#pragma unroll
+  for (int q = 0; q < K + 2; ++q) w[q] = W[l + q];
+#pragma unroll
+  for (int q = 0; q < K + 1; ++q) s[q] = S[l + q];
+#pragma unroll
+  for (int q = 0; q < K + 1; ++q) d[q] = D[l + q];
+  bool ok = (x[0] >= w[0]) & (x[0] < w[1]) & (x[3] < w[K + 1]);  // segment 0 holds the first bin
+  P[0] = s[0] + (x[0] - w[0]) * d[0];
+#pragma unroll
+  for (int t = 1; t < 4; ++t) {
+    float wl = w[0], sv = s[0], dv = d[0];
+#pragma unroll
+    for (int q = 1; q <= (t < K ? t : K); ++q) {
+      const bool in = x[t] >= w[q];
+      wl = in ? w[q] : wl;
+      sv = in ? s[q] : sv;
+      dv = in ? d[q] : dv;
+    }
+    if (t < K) ok &= x[t] < w[t + 1];
+    P[t] = sv + (x[t] - wl) * dv;
+  }
+  return ok;
+}
+
+// P of one bin of a staged window from any starting segment: the exact search
+// with the grid-end bounds and clamps of win_values<NB, false>.
+__device__ inline float window_value(float x, int l, int k_lo, int nk, int n_wave, const float* W,
+                                     const float* S) {
+  l = l < 0 ? 0 : (l > nk - 2 ? nk - 2 : l);
+  while (l < nk - 2 && l + k_lo + 1 < n_wave - 1 && x >= W[l + 1]) ++l;
+  while (l > 0 && x < W[l]) --l;
+  const float wl = W[l], wr = W[l + 1], s0 = S[l], s1 = S[l + 1];
+  const float dx = wr - wl;
+  const int i = l + k_lo + 1;  // global right knot
+  float th = (x - wl) * __builtin_amdgcn_rcpf(dx);
+  th = (i == 1 && x < wl) ? 0.f : ((i == n_wave - 1 && x > wr) ? 1.f : (dx > 0.f ? th : 0.f));
+  return s0 + th * (s1 - s0);
+}
+
+// The per-star constants of the forward, wave-uniform.
+struct StarVals {
+  int row;
+  float a, inv_a, m, T, av;
+  float w[4];
+};
+
+// Stage the window [k_lo, k_lo + nk) of runs, one knot per lane, 63 new ones a
+// round: shifted knots W (as the reference's wave * a), S_k = F_k m (rounded
+// once per knot as the reference's spectra) and slopes D.  The last knot's
+// slope is not used.
+__device__ inline void stage_run(const SspView& g, const Rows& R, const StarVals& s, int k_lo, int nk,
+                                 int lane, float* W, float* S, float* D) {
+  for (int b = 0; b < nk - 1; b += 63) {
+    const int k = b + lane;
+    const uint32_t kk = uint32_t(k_lo + (k < nk ? k : nk - 1));
+    const float lw = ld_at(g.wave, kk);
+    float fc[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) fc[c] = ld_at(R.f[c], kk);
+    __builtin_amdgcn_sched_group_barrier(0x020, 5, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+    float f = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f += s.w[c] * fc[c];
+    const float w = mul_nocontract(lw, s.a), v = f * s.m;
+    const float d = (next_lane(v) - v) * __builtin_amdgcn_rcpf(next_lane(w) - w);
+    if (k < nk) {
+      W[k] = w;
+      S[k] = v;
+      if (lane < 63) D[k] = d;
+    }
+  }
+}
+
+// P of a lane's runs for one star: run r is the four bins at xs[256 r + 4 lane].
+// The window's density picks how many segments a run may span: with evenly
+// spread knots, at most 0.33 per bin put a run of four bins into 2 segments,
+// at most 0.66 into 3.  The rest (a window at a grid end or over kRunKnots, a
+// bin outside its candidates) is done bin by bin.
+template <int kRuns>
+__device__ inline void run_values(const SspView& g, const StarVals& s, const float* xs, float x_last,
+                                  int lane, float* W, float* S, float* D, float (&P)[4 * kRuns]) {
+  const Rows R = rows_of(g, s.row);
+  const Shift h = shift_of(g, s.a, s.inv_a);
+  int k0[kRuns];
+#pragma unroll
+  for (int r = 0; r < kRuns; ++r) k0[r] = loc_k0(g, xs[256 * r + 4 * lane], h);
+  const int kl = loc_k0(g, x_last, h);
+  const int lo = __builtin_amdgcn_readfirstlane(k0[0]) - 3;
+  const int hi = __builtin_amdgcn_readfirstlane(kl) + 5;
+  const int k_lo = lo < 0 ? 0 : lo;
+  const int nk = (hi > g.n_wave - 1 ? g.n_wave - 1 : hi) - k_lo + 1;
+  const bool staged = nk <= kRunKnots;
+  bool ok = false;
+  if (staged) {
+    stage_run(g, R, s, k_lo, nk, lane, W, S, D);
+    wave_lds_sync();
+    if (k_lo >= 1 && k_lo + nk < g.n_wave) {  // no segment touches a grid end
+      ok = true;
+#pragma unroll
+      for (int r = 0; r < kRuns; ++r) {
+        const float4 xv = *reinterpret_cast<const float4*>(xs + 256 * r + 4 * lane);
+        const float x[4] = {xv.x, xv.y, xv.z, xv.w};
+        if (nk <= 84 * kRuns + 9) ok &= run_segments<1>(x, k0[r] - k_lo, W, S, D, P + 4 * r);
+        else ok &= run_segments<2>(x, k0[r] - k_lo, W, S, D, P + 4 * r);
+      }
+    }
+  }
+  if (__ballot(!ok)) {
+    StarState st;
+    st.m = s.m;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) st.w[c] = s.w[c];
+#pragma unroll
+    for (int r = 0; r < kRuns; ++r) {
+#pragma unroll 1
+      for (int t = 0; t < 4; ++t) {
+        const float xt = xs[256 * r + 4 * lane + t];
+        const float v = staged ? window_value(xt, k0[r] - k_lo, k_lo, nk, g.n_wave, W, S)
+                               : star_value(R, st, knots_of<false>(g, xt, h));
+        P[4 * r] = t == 0 ? v : P[4 * r];
+        P[4 * r + 1] = t == 1 ? v : P[4 * r + 1];
+        P[4 * r + 2] = t == 2 ? v : P[4 * r + 2];
+        P[4 * r + 3] = t == 3 ? v : P[4 * r + 3];
+      }
+    }
+  }
+  wave_lds_sync();  // this window's reads done before the next star's stores
+}
+
+// P of a lane's NB strided bins for one star.
+template <int NB>
+__device__ inline void strided_values(const SspView& g, const rbx_target& tg, const StarVals& sv,
+                                      const float* xs, uint32_t jh, uint32_t jh_end, int lane,
+                                      float* W, float* S, float (&P)[NB]) {
   constexpr int kHalfWindow = fused_window<NB>();
-  __shared__ float W_s[kFusedWaves][kHalfWindow];  // shifted knots of each wavefront's window
-  __shared__ float S_s[kFusedWaves][kHalfWindow];  // the star's spectrum at those knots
-  __shared__ float4 st_s[4 * kStateBatch];
-  __shared__ float nn_s[2][2][4 * kFusedWaves];  // [buffer][star of the pair][share]
-  __shared__ float x_s[kFusedWaves][NB][64];   // the lanes' target wavelengths
-  __shared__ float dt_s[kFusedWaves][NB][64];  // and bin widths
+  const Rows R = rows_of(g, sv.row);
+  const Shift h = shift_of(g, sv.a, sv.inv_a);
+  int k0[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t) k0[t] = loc_k0(g, xs[64 * t + lane], h);
+  int k_lo, nk;
+  if (!g.loc_multi) {
+    // the guesses are monotone in x: lane 0's first and lane 63's
+    // last bin bound the wavefront's, widened by the error bound
+    const int lo = __builtin_amdgcn_readfirstlane(k0[0]) - 3;
+    const int hi = __builtin_amdgcn_readlane(k0[NB - 1], 63) + 5;
+    k_lo = lo < 0 ? 0 : lo;
+    nk = (hi > g.n_wave - 1 ? g.n_wave - 1 : hi) - k_lo + 1;
+  } else {
+    slab_window(g, tg, jh, jh_end, h, &k_lo, &nk);
+  }
+  if (nk <= kHalfWindow) {
+    // shifted knot as the reference's wave * a; S_k = F_k m,
+    // rounded once per knot as the reference's spectra
+    if (nk > 128) {
+      // wide windows (knots denser than the bins): four knots per
+      // lane in 16-byte loads, one round of loads up to 256 knots.
+      // The last group ends on the window's last knot (b = nk - 4),
+      // so no load leaves the grid; its knots overlap the lane
+      // before, which stores the same values.
+      for (int k = 4 * lane; k < nk; k += 256) {
+        const int b = k + 4 <= nk ? k : nk - 4;
+        const uint32_t kk = uint32_t(k_lo + b);
+        const Quad lw = ld_quad(g.wave, kk);
+        Quad fc[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fc[c] = ld_quad(R.f[c], kk);
+        // the five loads in flight together, then the arithmetic
+        __builtin_amdgcn_sched_group_barrier(0x020, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float f = 0.f;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) f += sv.w[c] * fc[c].v[e];
+          W[b + e] = mul_nocontract(lw.v[e], sv.a);
+          S[b + e] = f * sv.m;
+        }
+      }
+    } else {
+      // narrow windows: one knot per lane (a quarter of the
+      // arithmetic per round when the window fits 64 or 128 lanes)
+      for (int k = lane; k < nk; k += 64) {
+        const uint32_t kk = uint32_t(k_lo + k);
+        const float lw = ld_at(g.wave, kk);
+        float fc[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fc[c] = ld_at(R.f[c], kk);
+        __builtin_amdgcn_sched_group_barrier(0x020, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+        float f = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) f += sv.w[c] * fc[c];
+        W[k] = mul_nocontract(lw, sv.a);
+        S[k] = f * sv.m;
+      }
+    }
+    wave_lds_sync();
+    float x[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) x[t] = xs[64 * t + lane];
+    // every bin of the lane, also one past the end (its x lies in the window)
+    if (k_lo >= 1 && k_lo + nk < g.n_wave && !g.loc_multi)
+      win_values<NB, true>(x, k0, k_lo, nk, g.n_wave, W, S, P);
+    else
+      win_values<NB, false>(x, k0, k_lo, nk, g.n_wave, W, S, P);
+    wave_lds_sync();  // this window's reads done before the next star's stores
+  } else {
+    StarState s;
+    s.m = sv.m;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s.w[c] = sv.w[c];
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      if (jh + lane + 64u * t < jh_end)
+        P[t] = star_value(R, s, knots_of<false>(g, xs[64 * t + lane], h));
+    }
+  }
+}
+
+// Workgroups of at most kWaves wavefronts (at least ceil(n / 64 NB)):
+// short axes take small workgroups, several to a CU.  kRuns > 0: that many
+// runs of four bins per lane (NB = 4 kRuns); kRuns = 0: NB strided bins.
+// Runs, and up to 4 strided bins per lane, hold to 64 VGPRs (8 wavefronts per
+// SIMD); more strided bins take 128 (4 per SIMD).
+// Bound by VALU issue with runs (84 % of the slots).
+template <bool kDust, int NB, int kWaves, int kRuns>
+__global__ void __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(kRuns > 0 || NB <= 4 ? 8 : 4)))
+cube_fused_kernel(SspView g, rbx_target tg, const StarState* __restrict__ stars,
+                  StarState* state, const ChunkDesc* __restrict__ desc,
+                  const int32_t* __restrict__ n_chunks_ptr, int64_t n_items,
+                  const float* __restrict__ axav, double* __restrict__ partial) {
+  static_assert(kRuns == 0 || NB == 4 * kRuns, "runs of four bins");
+  constexpr bool kRun = kRuns > 0;
+  // per wavefront: windows W, S (and D with runs), then the bins' wavelengths
+  // (and widths when strided)
+  constexpr int kWin = kRun ? kRunKnots : fused_window<NB>();
+  constexpr int kWinFloats = (kRun ? 3 : 2) * kWin;
+  static_assert(!kRun || kWinFloats * 4 >= 64 * 4 * 8, "a run's sums pass through the window space");
+  __shared__ __align__(16) float buf_s[kWaves][kWinFloats + (kRun ? 64 : 128) * NB];
+  // shares of Nn [buffer][star of the pair][share]: a total per wavefront with
+  // runs (fewer vector instructions), else four row sums (a shorter chain)
+  constexpr int kShares = kRun ? kFusedWaves : 4 * kFusedWaves;
+  __shared__ float nn_s[2][2][kShares];
+  __shared__ float4 st_s[kRun ? 1 : 4 * 64];  // strided: a batch of star records
   static_assert(sizeof(StarState) == 4 * sizeof(float4), "a star state is four float4");
   const int n_chunks = *n_chunks_ptr;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int slab = wave >> 1, half = wave & 1;
+  const int n_waves = int(blockDim.x >> 6);
   const int lane = threadIdx.x & 63;
-  float* W = W_s[wave];
-  float* S = S_s[wave];
-  const uint32_t j0 = uint32_t(slab * slab_bins);
-  const uint32_t j1 = j0 + slab_bins < uint32_t(tg.n) ? j0 + slab_bins : uint32_t(tg.n);
-  // this wavefront's bins [jh, jh_end)
-  const uint32_t jh = j0 + 64u * NB * half;
-  const uint32_t jh_end = jh + 64u * NB < j1 ? jh + 64u * NB : j1;
-  // the lane's bins, the same for every chunk: a bin past the end takes the
-  // last bin's x (inside the window) and weight 0, so it adds nothing to Nn
+  float* W = buf_s[wave];
+  float* S = W + kWin;
+  float* D = S + kWin;            // runs only
+  float* xs = W + kWinFloats;     // the lanes' target wavelengths
+  float* dts = xs + 64 * NB;      // and bin widths (strided only)
+  // this wavefront's bins [jh, jh_end), none for a wavefront past the axis
+  const uint32_t nt = uint32_t(tg.n);
+  const uint32_t jh = 64u * NB * uint32_t(wave);
+  const uint32_t jh_end = jh + 64u * NB < nt ? jh + 64u * NB : nt;
+  // shares of wavefronts that are not there stay 0
+  if (threadIdx.x < kShares && int(threadIdx.x) >= n_waves * (kShares / kFusedWaves))
+    for (int k = 0; k < 4; ++k) nn_s[k >> 1][k & 1][threadIdx.x] = 0.f;
+  const float x_last = uniform_f(ld_at(tg.wave, jh_end - 1));
+  // the lane's bin t, the same for every chunk: a bin past the end takes the
+  // last bin's x (inside the window) and width 0, so it adds nothing to Nn
   // and its sum is never stored.  x and the widths wait in LDS and are read
-  // where used (fewer registers live through the staging loop).
+  // where used (fewer registers live through the staging loop); a run's
+  // widths are the differences of its x.
+  auto slot_of = [&](int t) { return kRun ? 256 * (t >> 2) + 4 * lane + (t & 3) : 64 * t + lane; };
   float tau[NB];
 #pragma unroll
   for (int t = 0; t < NB; ++t) {
-    const uint32_t j = jh + lane + 64u * t;
-    const uint32_t jc = j < j1 ? j : (j1 > j0 ? j1 - 1 : 0);
+    const uint32_t j = jh + uint32_t(slot_of(t));
+    const uint32_t jc = j < jh_end ? j : jh_end - 1;
     const Pair xd = ld_pair(tg.pairs, 2 * jc);
-    x_s[wave][t][lane] = xd.lo;
-    dt_s[wave][t][lane] = j < jh_end ? xd.hi : 0.f;
+    xs[slot_of(t)] = xd.lo;
+    if (!kRun) dts[slot_of(t)] = j < jh_end ? xd.hi : 0.f;
     tau[t] = kDust ? dust_tau(axav, jc) : 0.f;
   }
+  // the bin before the wavefront's first (none before bin 0: width 0)
+  const float x_before = uniform_f(ld_at(tg.wave, jh > 0 && jh < nt ? jh - 1 : 0));
   for (int64_t q = blockIdx.x; q < n_items; q += gridDim.x) {
     if (q >= n_chunks) break;  // chunk count is uniform: the whole workgroup leaves
     const ChunkDesc d = desc[q];
@@ -825,22 +1102,31 @@ cube_fused_kernel(SspView g, rbx_target tg, StarState* __restrict__ state,
 #pragma unroll
     for (int t = 0; t < NB; ++t) acc[t] = 0.0;
     int par = 0;
-    for (int b0 = d.begin; b0 < d.end; b0 += kStateBatch) {
-      const int nb_st = d.end - b0 < kStateBatch ? d.end - b0 : kStateBatch;
-      __syncthreads();  // the previous batch's states are read
-      const float4* src = reinterpret_cast<const float4*>(state + b0);
-      for (int i = threadIdx.x; i < 4 * nb_st; i += 64 * kFusedWaves) st_s[i] = src[i];
-      __syncthreads();
-      // P_j of star i of the batch on this wavefront's bins; false (P = 0)
-      // for a dropped star (uniform: the same star for every wavefront)
-      auto star_values = [&](int i, float (&P)[NB], float& T, float& av) -> bool {
-        const float4 s0 = st_s[4 * i], s1 = st_s[4 * i + 1], s2 = st_s[4 * i + 2];
-        const int row = __builtin_amdgcn_readfirstlane(__float_as_int(s0.x));
+    // P_j of star r, the i-th of its batch, on this wavefront's bins; false
+    // (P = 0) for a dropped star (uniform: the same star for every wavefront).
+    // Runs read the record through the scalar cache (11 vector instructions
+    // fewer, sf and Nn not read), its row from the batch's load; the strided
+    // bins, which wait on latency, read it from LDS.
+    int rows = -1;
+    auto star_values = [&](int r, int i, float (&P)[NB], float& T, float& av) -> bool {
+      StarVals s;
 #pragma unroll
-        for (int t = 0; t < NB; ++t) P[t] = 0.f;
-        if (row < 0) return false;
-        StarState s;
-        s.row = row;
+      for (int t = 0; t < NB; ++t) P[t] = 0.f;
+      if constexpr (kRun) {
+        s.row = __builtin_amdgcn_readlane(rows, i);
+        if (s.row < 0) return false;
+        const StarState& st = stars[r];
+        s.a = st.a;
+        s.inv_a = st.inv_a;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s.w[c] = st.w[c];
+        s.m = st.m;
+        T = st.T;
+        av = kDust ? st.av : 0.f;
+      } else {
+        const float4 s0 = st_s[4 * i], s1 = st_s[4 * i + 1], s2 = st_s[4 * i + 2];
+        s.row = __builtin_amdgcn_readfirstlane(__float_as_int(s0.x));
+        if (s.row < 0) return false;
         s.a = uniform_f(s0.z);
         s.inv_a = uniform_f(s0.w);
         s.w[0] = uniform_f(s1.x);
@@ -850,137 +1136,97 @@ cube_fused_kernel(SspView g, rbx_target tg, StarState* __restrict__ state,
         s.m = uniform_f(s2.x);
         T = uniform_f(s2.y);
         av = kDust ? uniform_f(st_s[4 * i + 3].w) : 0.f;
-        if (jh < jh_end) {
-          const Rows R = rows_of(g, s.row);
-          const Shift h = shift_of(g, s.a, s.inv_a);
-          int k0[NB];
+      }
+      if (jh >= jh_end) return true;
+      if constexpr (kRun) run_values<kRuns>(g, s, xs, x_last, lane, W, S, D, P);
+      else strided_values<NB>(g, tg, s, xs, jh, jh_end, lane, W, S, P);
+      return true;
+    };
+    // this wavefront's share of Nn = sum_j P_j dtarget_j
+    auto post_share = [&](const float (&P)[NB], float* slot) {
+      float nn = 0.f;
+      if constexpr (kRun) {
+        float before = x_before;
 #pragma unroll
-          for (int t = 0; t < NB; ++t) k0[t] = loc_k0(g, x_s[wave][t][lane], h);
-          int k_lo, nk;
-          if (!g.loc_multi) {
-            // the guesses are monotone in x: lane 0's first and lane 63's
-            // last bin bound the wavefront's, widened by the error bound
-            const int lo = __builtin_amdgcn_readfirstlane(k0[0]) - 3;
-            const int hi = __builtin_amdgcn_readlane(k0[NB - 1], 63) + 5;
-            k_lo = lo < 0 ? 0 : lo;
-            nk = (hi > g.n_wave - 1 ? g.n_wave - 1 : hi) - k_lo + 1;
-          } else {
-            slab_window(g, tg, jh, jh_end, h, &k_lo, &nk);
-          }
-          if (nk <= kHalfWindow) {
-            // shifted knot as the reference's wave * a; S_k = F_k m,
-            // rounded once per knot as the reference's spectra
-            if (nk > 128) {
-              // wide windows (knots denser than the bins): four knots per
-              // lane in 16-byte loads, one round of loads up to 256 knots.
-              // The last group ends on the window's last knot (b = nk - 4),
-              // so no load leaves the grid; its knots overlap the lane
-              // before, which stores the same values.
-              for (int k = 4 * lane; k < nk; k += 256) {
-                const int b = k + 4 <= nk ? k : nk - 4;
-                const uint32_t kk = uint32_t(k_lo + b);
-                const Quad lw = ld_quad(g.wave, kk);
-                Quad fc[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) fc[c] = ld_quad(R.f[c], kk);
-                // the five loads in flight together, then the arithmetic
-                __builtin_amdgcn_sched_group_barrier(0x020, 5, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  float f = 0.f;
-#pragma unroll
-                  for (int c = 0; c < 4; ++c) f += s.w[c] * fc[c].v[e];
-                  W[b + e] = mul_nocontract(lw.v[e], s.a);
-                  S[b + e] = f * s.m;
-                }
-              }
-            } else {
-              // narrow windows: one knot per lane (a quarter of the
-              // arithmetic per round when the window fits 64 or 128 lanes)
-              for (int k = lane; k < nk; k += 64) {
-                const uint32_t kk = uint32_t(k_lo + k);
-                const float lw = ld_at(g.wave, kk);
-                float fc[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) fc[c] = ld_at(R.f[c], kk);
-                __builtin_amdgcn_sched_group_barrier(0x020, 5, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-                float f = 0.f;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) f += s.w[c] * fc[c];
-                W[k] = mul_nocontract(lw, s.a);
-                S[k] = f * s.m;
-              }
-            }
-            wave_lds_sync();
-            float x[NB];
-#pragma unroll
-            for (int t = 0; t < NB; ++t) x[t] = x_s[wave][t][lane];
-            // every bin of the lane, also one past the end (its x lies in the window)
-            if (k_lo >= 1 && k_lo + nk < g.n_wave && !g.loc_multi)
-              win_values<NB, true>(x, k0, k_lo, nk, g.n_wave, W, S, P);
-            else
-              win_values<NB, false>(x, k0, k_lo, nk, g.n_wave, W, S, P);
-            wave_lds_sync();  // this window's reads done before the next star's stores
-          } else {
-#pragma unroll
-            for (int t = 0; t < NB; ++t) {
-              if (jh + lane + 64u * t < jh_end) {
-                const Knots K = knots_of<false>(g, x_s[wave][t][lane], h);
-                P[t] = star_value(R, s, K);
-              }
-            }
-          }
+        for (int q4 = 0; q4 < kRuns; ++q4) {
+          const float4 x = *reinterpret_cast<const float4*>(xs + 256 * q4 + 4 * lane);
+          nn += P[4 * q4] * (x.x - prev_lane(x.w, before));
+          nn += P[4 * q4 + 1] * (x.y - x.x);
+          nn += P[4 * q4 + 2] * (x.z - x.y);
+          nn += P[4 * q4 + 3] * (x.w - x.z);
+          if (q4 + 1 < kRuns) before = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x.w), 63));
         }
-        return true;
-      };
-      // this wavefront's four row sums of Nn = sum_j P_j dtarget_j
-      auto post_share = [&](const float (&P)[NB], float* slot) {
-        float nn = 0.f;
+      } else {
 #pragma unroll
-        for (int t = 0; t < NB; ++t) nn += P[t] * dt_s[wave][t][lane];
+        for (int t = 0; t < NB; ++t) nn += P[t] * dts[64 * t + lane];
+      }
+      if constexpr (kRun) {
+        nn = wave_sum_last(nn);
+        if (lane == 63) slot[wave] = nn;
+      } else {
         nn = row_sum16(nn);
         if ((lane & 15) == 0) slot[4 * wave + (lane >> 4)] = nn;
-      };
-      // sf = nan_to_num(T / Nn) from the 64 shares (added in a fixed order),
-      // stored for the adjoint, and P_j sf into the f64 sums
-      auto accumulate = [&](const float (&P)[NB], float T, float av, const float* slot, int r) {
-        const float Nn = wave_sum_dpp(slot[lane]);
-        // T / Nn with the hardware reciprocal (within one ulp of the division;
-        // Nn = 0 still gives inf or nan for nan_to_num below)
-        float sf = T * __builtin_amdgcn_rcpf(Nn);
-        if (isnan(sf)) sf = 0.f;
-        else if (isinf(sf)) sf = sf > 0.f ? FLT_MAX : -FLT_MAX;
-        if (wave == 0 && lane == 0) {
-          state[r].sf = sf;
-          state[r].Nn = Nn;
-        }
+      }
+    };
+    // sf = nan_to_num(T / Nn) from the shares (added in a fixed order),
+    // stored for the adjoint, and P_j sf into the f64 sums
+    auto accumulate = [&](const float (&P)[NB], float T, float av, const float* slot, int r) {
+      const float Nn = kRun ? row_sum16(slot[lane & (kFusedWaves - 1)]) : wave_sum_dpp(slot[lane & (kShares - 1)]);
+      // T / Nn with the hardware reciprocal (within one ulp of the division;
+      // Nn = 0 still gives inf or nan for nan_to_num)
+      const float q0 = T * __builtin_amdgcn_rcpf(Nn);
+      const float sf = isnan(q0) ? 0.f : fminf(fmaxf(q0, -FLT_MAX), FLT_MAX);
+      if (wave == 0 && lane == 0) {
+        state[r].sf = sf;
+        state[r].Nn = Nn;
+      }
 #pragma unroll
-        for (int t = 0; t < NB; ++t) {
-          float v = P[t] * sf;
-          if (kDust && av != 0.f) v *= dust_factor(tau[t], av);
-          acc[t] += double(v);
+      for (int t = 0; t < NB; ++t) {
+        float v = P[t] * sf;
+        if (kDust && av != 0.f) v *= dust_factor(tau[t], av);
+        acc[t] += double(v);
+      }
+    };
+    // two stars per barrier: both stars' shares are posted, then one
+    // barrier; the stars are added in order as one at a time would
+    for (int r = d.begin; r < d.end; r += 2) {
+      const int i = (r - d.begin) & 63;
+      if (i == 0) {  // the next batch of 64 stars
+        if constexpr (kRun) {
+          rows = r + lane < d.end ? stars[r + lane].row : -1;
+        } else {
+          const int nb_st = d.end - r < 64 ? d.end - r : 64;
+          __syncthreads();  // the previous batch's states are read
+          const float4* src = reinterpret_cast<const float4*>(stars + r);
+          for (int k = threadIdx.x; k < 4 * nb_st; k += int(blockDim.x)) st_s[k] = src[k];
+          __syncthreads();
         }
-      };
-      // two stars per barrier: both stars' shares are posted, then one
-      // barrier; the stars are added in batch order as one at a time would
-      for (int i = 0; i < nb_st; i += 2) {
-        float PA[NB], PB[NB];
-        float TA = 0.f, TB = 0.f, avA = 0.f, avB = 0.f;
-        const bool va = star_values(i, PA, TA, avA);
-        const bool vb = i + 1 < nb_st && star_values(i + 1, PB, TB, avB);
-        if (!va && !vb) continue;
-        if (!vb) {
+      }
+      float PA[NB], PB[NB];
+      float TA = 0.f, TB = 0.f, avA = 0.f, avB = 0.f;
+      const bool va = star_values(r, i, PA, TA, avA);
+      const bool vb = r + 1 < d.end && star_values(r + 1, i + 1, PB, TB, avB);
+      if (!va && !vb) continue;
+      if (!vb) {
 #pragma unroll
-          for (int t = 0; t < NB; ++t) PB[t] = 0.f;
-        }
-        post_share(PA, nn_s[par][0]);
-        post_share(PB, nn_s[par][1]);
-        __syncthreads();  // every share of both stars posted
-        if (va) accumulate(PA, TA, avA, nn_s[par][0], b0 + i);
-        if (vb) accumulate(PB, TB, avB, nn_s[par][1], b0 + i + 1);
-        par ^= 1;
+        for (int t = 0; t < NB; ++t) PB[t] = 0.f;
+      }
+      post_share(PA, nn_s[par][0]);
+      post_share(PB, nn_s[par][1]);
+      __syncthreads();  // every share of both stars posted
+      if (va) accumulate(PA, TA, avA, nn_s[par][0], r);
+      if (vb) accumulate(PB, TB, avB, nn_s[par][1], r + 1);
+      par ^= 1;
+    }
+    if constexpr (kRun) {
+      // through the wavefront's window space, so that the stores are contiguous
+      double* sums = reinterpret_cast<double*>(W);
+#pragma unroll
+      for (int q4 = 0; q4 < kRuns; ++q4) {
+        for (int t = 0; t < 4; ++t) sums[4 * lane + t] = acc[4 * q4 + t];
+        wave_lds_sync();
+        for (int t = 0; t < 4; ++t) acc[4 * q4 + t] = sums[64 * t + lane];
+        wave_lds_sync();
       }
     }
 #pragma unroll
@@ -1172,11 +1418,6 @@ __global__ void __launch_bounds__(64 * W) star_bwd_kernel(
 // v of lane l (0 <= l < 64) by one ds_bpermute (no lane wrapping needed).
 __device__ inline float lane_of(float v, int l) {
   return __int_as_float(__builtin_amdgcn_ds_bpermute(l << 2, __float_as_int(v)));
-}
-
-// The next lane's v (DPP wave shift left by one); lane 63 reads 0.
-__device__ inline float next_lane(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
 }
 
 // Change of the combined row R_w from this lane's knot to the next lane's,
@@ -1844,6 +2085,30 @@ void combine_chunks(const double* partial, const int32_t* chunk_off, int32_t ns,
                      partial, chunk_off, ns, bands, nt, cube);
 }
 
+// Wavefronts of a fused workgroup: 64 NB bins each.
+static int fused_waves(int nt, int nb) { return (nt + 64 * nb - 1) / (64 * nb); }
+
+// Runs where the smallest knot spacing (1 / locate_inv_h on a locator with one
+// knot per cell) is at least 2.25 times the mean bin spacing: 512 bins then
+// span at most 237 knots with the margins.
+static bool fused_runs(const rbx_ssp& ssp, const rbx_target& tg) {
+  return !ssp.locate_multi && tg.n > 1 &&
+         float(tg.n - 1) >= 2.25f * ssp.locate_inv_h * (tg.wmax - tg.wmin);
+}
+
+// Stars per reduction chunk where the caller leaves it open.  A chunk's stars
+// are walked one after another (about 1 us each), so the largest chunk is the
+// tail of the launch: eight chunks for every resident workgroup (2 of 16
+// wavefronts a CU, 4 of 8, 7 of 4) keep it short, at the price of one f64
+// partial row per chunk.  At 10 k stars -> 25 x 25 x 1000 chunks of up to 256
+// took 183 us, one spaxel at the field's edge holding most of that; now 26 us.
+static int auto_chunk(int64_t n, int32_t nt) {
+  const int w = fused_waves(nt < 4096 ? nt : 4096, 4);
+  const int64_t slots = 256 * (w > 8 ? 2 : (w > 4 ? 4 : 7));  // of the chip's 256 CUs
+  const int64_t c = n / (8 * slots);
+  return c < 8 ? 8 : (c > 256 ? 256 : int(c));
+}
+
 size_t cube_workspace_impl(int64_t n, int32_t n_keys, int32_t nt, const Tune& t) {
   if (n < 0 || n_keys < 1 || nt < 1) return 0;
   SizeOnly so;
@@ -1859,22 +2124,24 @@ struct FusedLaunch {
   StarState* state;
   const ChunkDesc* desc;
   const int32_t* n_chunks;
-  int slab_bins;
   int64_t items;
   const float* axav;
   double* partial;
 };
 
-template <int NB>
+template <int NB, int kWaves, int kRuns = 0>
 void launch_fused(const FusedLaunch& f) {
+  // whole rounds of the 4 SIMDs above 4 wavefronts: 15 of 16 put two
+  // workgroups' odd ones on the same SIMD (6.6 against 6.15 ms at 1 M stars)
+  const int need = fused_waves(f.tg.n, NB);
+  const int waves = need <= 4 ? need : (need + 3) / 4 * 4;
+  const dim3 block(64 * unsigned(waves));
   if (f.axav)
-    hipLaunchKernelGGL((cube_fused_kernel<true, NB>), dim3(f.grid), dim3(64 * kFusedWaves), 0,
-                       f.s, f.g, f.tg, f.state, f.desc, f.n_chunks, f.slab_bins, f.items, f.axav,
-                       f.partial);
+    hipLaunchKernelGGL((cube_fused_kernel<true, NB, kWaves, kRuns>), dim3(f.grid), block, 0, f.s, f.g, f.tg,
+                       f.state, f.state, f.desc, f.n_chunks, f.items, f.axav, f.partial);
   else
-    hipLaunchKernelGGL((cube_fused_kernel<false, NB>), dim3(f.grid), dim3(64 * kFusedWaves), 0,
-                       f.s, f.g, f.tg, f.state, f.desc, f.n_chunks, f.slab_bins, f.items,
-                       nullptr, f.partial);
+    hipLaunchKernelGGL((cube_fused_kernel<false, NB, kWaves, kRuns>), dim3(f.grid), block, 0, f.s, f.g,
+                       f.tg, f.state, f.state, f.desc, f.n_chunks, f.items, nullptr, f.partial);
 }
 
 int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars* stars,
@@ -1907,7 +2174,8 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   // ascending targets with at most kMaxFusedBins bins per lane: one fused
   // pass (cube_fused_kernel, NB bins per lane); otherwise (or when the
   // tuning asks for it) star_norm + star_sf, then the per-tile accumulation
-  const int nb_lane = (tps + 1) / 2 < 4 ? 4 : (tps + 1) / 2;
+  const int nb_need = (n_tiles + kFusedWaves - 1) / kFusedWaves;
+  const int nb_lane = nb_need < 4 ? 4 : nb_need;
   const bool fused = target->ascending && nb_lane <= kMaxFusedBins &&
                      !(t.flags & RBX_TUNE_TWO_PASS);
   if (n > 0) {
@@ -1934,13 +2202,23 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
     const int64_t items = L.max_chunks;
     const int64_t grid = item_grid(items, t.persist, 64 * kFusedWaves);
     const FusedLaunch f{grid, s, g, *target, L.state, L.desc, L.chunk_off + n_band_keys,
-                        tps * kTile, items, axav, L.partial};
-    switch (nb_lane) {
-      case 4: launch_fused<4>(f); break;
-      case 5: launch_fused<5>(f); break;
-      case 6: launch_fused<6>(f); break;
-      case 7: launch_fused<7>(f); break;
-      default: launch_fused<8>(f);
+                        items, axav, L.partial};
+    const int w = fused_waves(nt, 4), wr = fused_waves(nt, 8);
+    if (fused_runs(*ssp, *target)) {
+      if (wr <= 2) launch_fused<8, 2, 2>(f);
+      else if (wr <= 4) launch_fused<8, 4, 2>(f);
+      else if (wr <= 8) launch_fused<8, 8, 2>(f);
+      else launch_fused<8, 16, 2>(f);
+    } else switch (nb_lane) {
+      case 4:
+        if (w <= 4) launch_fused<4, 4>(f);
+        else if (w <= 8) launch_fused<4, 8>(f);
+        else launch_fused<4, 16>(f);
+        break;
+      case 5: launch_fused<5, 16>(f); break;
+      case 6: launch_fused<6, 16>(f); break;
+      case 7: launch_fused<7, 16>(f); break;
+      default: launch_fused<8, 16>(f);
     }
     if ((rc = check_launch(who))) return rc;
   } else if (n > 0) {
@@ -2017,6 +2295,7 @@ int rbx_ssp_prepare(const rbx_ssp* ssp, double* cum_out, int32_t* locate_out, vo
 size_t rbx_cube_workspace_size(int64_t n, int32_t n_keys, int32_t n_target) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
+  t.chunk = rbx::auto_chunk(n, n_target);
   return rbx::cube_workspace_impl(n, n_keys, n_target, t);
 }
 
@@ -2024,6 +2303,7 @@ int rbx_cube_fwd(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars* 
                  float* cube, void* workspace, size_t workspace_bytes, void* stream) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
+  if (stars && target) t.chunk = rbx::auto_chunk(stars->n, target->n);
   return rbx::cube_fwd_impl(ssp, target, stars, nullptr, t, cube, workspace, workspace_bytes,
                             rbx::as_stream(stream), "rbx_cube_fwd");
 }
@@ -2033,6 +2313,7 @@ int rbx_cube_fwd_ext(const rbx_ssp* ssp, const rbx_target* target, const rbx_sta
                      size_t workspace_bytes, void* stream) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
+  if (stars && target) t.chunk = rbx::auto_chunk(stars->n, target->n);
   return rbx::cube_fwd_impl(ssp, target, stars, ext, t, cube, workspace, workspace_bytes,
                             rbx::as_stream(stream), "rbx_cube_fwd_ext");
 }
