@@ -728,7 +728,7 @@ constexpr int kMaxFusedBins = 8;
 // wavefront stores sf and Nn for the adjoint.
 //
 // The bins of a lane:
-// * runs (run_values; knots well sparser than the bins, fused_runs()): kRuns
+// * runs (run_values; knots well sparser than the bins, sparse_knots()): kRuns
 //   runs of four consecutive bins.  One locator probe and one exact next-knot
 //   test place a run's first bin in its segment; the others lie in that
 //   segment or the one or two after it, whose left knots, values and slopes
@@ -1745,6 +1745,194 @@ __global__ void __launch_bounds__(64 * W) star_bwd_reg_kernel(
   }
 }
 
+// star_bwd_reg_kernel for sparse knots (sparse_knots()): blocks of 256
+// consecutive bins, a run of four per lane as in the forward.  The block's
+// knots are loaded one per lane, combined there and written to the
+// wavefront's LDS as records {w, R_w, dR_w/dw, R_u | dR_u/dw, R_s, dR_s/dw}
+// (slopes per shifted knot, the change of R_w from the corners' own
+// differences, w_change); a lane reads the records of its run's first segment
+// and of the one or two after it, and compares pick each bin's.  A knot is
+// thus loaded and combined once per 256 bins instead of once per 64 and the
+// cross-lane permutes (8 per bin) go: at 5.6 bins per knot 65 -> 43 vector
+// instructions per bin, 58.2 -> 36.5 ms at 10 M stars -> 3721 bins (VALU issue
+// in 93 % of the cycles).  Blocks at a grid end, wider than the record
+// space, or with a bin outside its candidates are gathered bin by bin.
+constexpr int kBwdRunBins = 256;
+constexpr int kBwdRunKnots = 126;  // two rounds of 63 and the last
+
+// The record space: one array per field, so that lanes on neighbouring knots
+// read without bank conflicts (32-byte records read 16 bytes at a time spent
+// 40 % of the kernel waiting on LDS).
+enum RunField { kRw, kRRw, kRSw, kRRu, kRSu, kRRs, kRSs, kRunFields };
+
+// The run's seven sums from the records at l (its first bin's segment, or one
+// before); false (nothing added) where a bin lies outside its candidates.
+template <int K>
+__device__ inline bool bwd_run(const float* rec, int l, const float (&x)[4], const float (&gj)[4],
+                               const float (&dj)[4], float v[7]) {
+  l += rec[l + 1] <= x[0] ? 1 : 0;
+  float a[kRunFields][K + 1];
+#pragma unroll
+  for (int f = 0; f < kRunFields; ++f) {
+#pragma unroll
+    for (int q = 0; q < K + 1; ++q) a[f][q] = rec[f * kBwdRunKnots + l + q];
+  }
+  const float w_end = rec[l + K + 1];
+  bool ok = (x[0] >= a[kRw][0]) & (x[0] < a[kRw][1]) & (x[3] < w_end);
+  if (K == 2) ok &= x[1] < a[kRw][K];  // bin 1 among the first two segments
+  if (__ballot(!ok)) return false;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float r[kRunFields];
+#pragma unroll
+    for (int f = 0; f < kRunFields; ++f) r[f] = a[f][0];
+#pragma unroll
+    for (int q = 1; q <= (t < K ? t : K); ++q) {
+      const bool in = x[t] >= a[kRw][q];
+#pragma unroll
+      for (int f = 0; f < kRunFields; ++f) r[f] = in ? a[f][q] : r[f];
+    }
+    const float d = x[t] - r[kRw];
+    const float Ruv = r[kRRu] + d * r[kRSu];
+    const float Rsv = r[kRRs] + d * r[kRSs];
+    v[0] += gj[t] * (r[kRRw] + d * r[kRSw]);
+    v[1] += gj[t] * Ruv;
+    v[2] += gj[t] * Rsv;
+    v[3] += dj[t] * Ruv;
+    v[4] += dj[t] * Rsv;
+    const float kd = x[t] * r[kRSw];  // a lambda(x) dR_w/dw: lambda(x) = x / a, 1 / a after the last bin
+    v[5] -= gj[t] * kd;
+    v[6] -= dj[t] * kd;
+  }
+  return true;
+}
+
+template <int W, bool kDust>
+__global__ void __launch_bounds__(64 * W) star_bwd_run_kernel(
+    SspView g, rbx_target tg, int64_t n, int64_t n_items, const StarState* __restrict__ state,
+    const float* __restrict__ gradw, const float* __restrict__ dcube, int slab_bins,
+    const float* __restrict__ axav, float* __restrict__ vpart, double* __restrict__ apart) {
+  constexpr int kBuf = kRunFields * kBwdRunKnots + 2;  // a multiple of 16 bytes
+  static_assert(kBuf >= kRedFloats, "the lane sums reuse the record space");
+  __shared__ __align__(16) float buf_s[W][kBuf];
+  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const SlabTask t = slab_task<W, kBwdSlabs>(item);
+    const bool live = t.r < n;
+    float* buf = buf_s[t.wave];
+    float v[7];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) v[q] = 0.f;
+    StarState s;
+    s.row = -1;
+    if (live) s = state[t.r];
+    if (s.row >= 0) {
+      const Rows R = rows_of(g, __builtin_amdgcn_readfirstlane(s.row));
+      const float* grow = dcube + int64_t(__builtin_amdgcn_readfirstlane(s.spaxel)) * tg.n;
+      s.a = uniform_f(s.a);
+      s.inv_a = uniform_f(s.inv_a);
+      const Shift h = shift_of(g, s.a, s.inv_a);
+      BwdRows B;
+      B.fu = uniform_f(gradw[t.r * 2]);
+      B.fs = uniform_f(gradw[t.r * 2 + 1]);
+      float wc[4];  // the corner weights, wave-uniform
+#pragma unroll
+      for (int c = 0; c < 4; ++c) wc[c] = uniform_f(s.w[c]);
+      const uint32_t j0 = uint32_t(t.slab * slab_bins);
+      const uint32_t j1 = j0 + slab_bins < uint32_t(tg.n) ? j0 + slab_bins : uint32_t(tg.n);
+      for (uint32_t jb = j0; jb < j1; jb += kBwdRunBins) {
+        const uint32_t j = jb + 4u * uint32_t(t.lane);
+        float x[4], dj[4], gj[4];
+        if (jb + kBwdRunBins <= j1) {
+          const Quad p0 = ld_quad(tg.pairs, 2 * j), p1 = ld_quad(tg.pairs, 2 * j + 4);
+          const Quad gq = ld_quad(grow, j);
+          x[0] = p0.v[0]; dj[0] = p0.v[1]; x[1] = p0.v[2]; dj[1] = p0.v[3];
+          x[2] = p1.v[0]; dj[2] = p1.v[1]; x[3] = p1.v[2]; dj[3] = p1.v[3];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) gj[q] = gq.v[q];
+        } else {
+          // bins past the slab take its last bin's x and weights 0
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const bool in = j + q < j1;
+            const uint32_t jc = in ? j + q : j1 - 1;
+            const Pair xd = ld_pair(tg.pairs, 2 * jc);
+            const float gv = ld_at(grow, jc);
+            x[q] = xd.lo;
+            dj[q] = in ? xd.hi : 0.f;
+            gj[q] = in ? gv : 0.f;
+          }
+        }
+        const int k0 = loc_k0(g, x[0], h);
+        const float x_last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x[3]), 63));
+        const int kl = loc_k0(g, x_last, h);
+        if (kDust && s.av != 0.f) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            gj[q] *= dust_factor(dust_tau(axav, j + q < j1 ? j + q : j1 - 1), s.av);
+        }
+        // every guess with a margin of 3 knots below and 5 above (run_values)
+        const int k_lo = __builtin_amdgcn_readfirstlane(k0) - 3;
+        const int nk = __builtin_amdgcn_readfirstlane(kl) + 5 - k_lo + 1;
+        bool done = false;
+        if (nk <= kBwdRunKnots && k_lo >= 1 && k_lo + nk < g.n_wave) {
+          wave_lds_sync();  // the block before is read
+          for (int b = 0; b < nk - 1; b += 63) {
+            const int k = b + t.lane;
+            const uint32_t kk = uint32_t(k_lo + (k < nk ? k : nk - 1));
+            const float lamk = ld_at(g.wave, kk);
+            float fc[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) fc[c] = ld_at(R.f[c], kk);
+            const RowVals rv = combine_rows(fc[0], fc[1], fc[2], fc[3], B.fu, B.fs);
+            const float dwk = w_change(fc, wc);
+            const float w = mul_nocontract(lamk, s.a);
+            const float r = __builtin_amdgcn_rcpf(next_lane(w) - w);
+            const float su = (next_lane(rv.u) - rv.u) * r, ss = (next_lane(rv.s) - rv.s) * r;
+            // lane 63 repeats the next round's first knot (its slopes need
+            // the knot after it); the window's last knot is only compared
+            if (k < nk && (t.lane < 63 || k == nk - 1)) {
+              buf[kRw * kBwdRunKnots + k] = w;
+              buf[kRRw * kBwdRunKnots + k] = rv.w;
+              buf[kRSw * kBwdRunKnots + k] = dwk * r;
+              buf[kRRu * kBwdRunKnots + k] = rv.u;
+              buf[kRSu * kBwdRunKnots + k] = su;
+              buf[kRRs * kBwdRunKnots + k] = rv.s;
+              buf[kRSs * kBwdRunKnots + k] = ss;
+            }
+          }
+          wave_lds_sync();
+          const int l = k0 - k_lo;  // in [3, nk - 6]: the guesses are monotone in the bin
+          done = nk <= 84 + 9 ? bwd_run<1>(buf, l, x, gj, dj, v)
+                              : bwd_run<2>(buf, l, x, gj, dj, v);
+        }
+        if (!done) {
+#pragma unroll 1
+          for (int q = 0; q < 4; ++q) {
+            const float xq = q == 0 ? x[0] : (q == 1 ? x[1] : (q == 2 ? x[2] : x[3]));
+            const float gq = q == 0 ? gj[0] : (q == 1 ? gj[1] : (q == 2 ? gj[2] : gj[3]));
+            const float dq = q == 0 ? dj[0] : (q == 1 ? dj[1] : (q == 2 ? dj[2] : dj[3]));
+            float u[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            bwd_bin_gather(g, R, s, B, h, xq, gq, dq, u);
+#pragma unroll
+            for (int e = 0; e < 5; ++e) v[e] += u[e];
+            v[5] += u[5] * s.a;
+            v[6] += u[6] * s.a;
+          }
+        }
+      }
+      v[5] *= s.inv_a;
+      v[6] *= s.inv_a;
+    }
+    const double tot = lds_sum<7>(v, buf, t.lane);
+    const int q = t.lane >> 3;
+    if (live && (t.lane & 7) == 0 && q < 7) {
+      const int64_t it = t.r * kBwdSlabs + t.slab;
+      if (q < kVSums) vpart[it * kVSums + q] = float(tot);
+      else apart[it * kASums + q - kVSums] = tot;
+    }
+  }
+}
+
 // Per star: add the slab sums in slab order and form every gradient in
 // closed form.  With P_j = m sum_c w_c R_c(j) and sf = T / Nn:
 //   sum_j g_j dP_j/dtheta = m Pg_theta, dNn/dtheta = m Pd_theta,
@@ -2028,7 +2216,16 @@ template <int W>
 static void launch_bwd(int64_t grid, hipStream_t s, const SspView& g, const rbx_target& tg,
                        int64_t n, int64_t items, const StarState* st, const float* gradw,
                        const float* dcube, int slab_bins, const float* axav, float* vp,
-                       double* ap) {
+                       double* ap, bool runs) {
+  if (runs) {
+    if (axav)
+      hipLaunchKernelGGL((star_bwd_run_kernel<W, true>), dim3(grid), dim3(64 * W), 0, s, g, tg, n,
+                         items, st, gradw, dcube, slab_bins, axav, vp, ap);
+    else
+      hipLaunchKernelGGL((star_bwd_run_kernel<W, false>), dim3(grid), dim3(64 * W), 0, s, g, tg,
+                         n, items, st, gradw, dcube, slab_bins, nullptr, vp, ap);
+    return;
+  }
   if (tg.ascending) {
     if (axav)
       hipLaunchKernelGGL((star_bwd_reg_kernel<W, true>), dim3(grid), dim3(64 * W), 0, s, g, tg, n,
@@ -2088,11 +2285,12 @@ void combine_chunks(const double* partial, const int32_t* chunk_off, int32_t ns,
 // Wavefronts of a fused workgroup: 64 NB bins each.
 static int fused_waves(int nt, int nb) { return (nt + 64 * nb - 1) / (64 * nb); }
 
-// Runs where the smallest knot spacing (1 / locate_inv_h on a locator with one
-// knot per cell) is at least 2.25 times the mean bin spacing: 512 bins then
-// span at most 237 knots with the margins.
-static bool fused_runs(const rbx_ssp& ssp, const rbx_target& tg) {
-  return !ssp.locate_multi && tg.n > 1 &&
+// Runs of bins (ascending targets) where the smallest knot spacing
+// (1 / locate_inv_h on a locator with one knot per cell) is at least 2.25 times
+// the mean bin spacing: 512 bins then span at most 237 knots with the
+// margins, 256 at most 123.
+static bool sparse_knots(const rbx_ssp& ssp, const rbx_target& tg) {
+  return tg.ascending && !ssp.locate_multi && tg.n > 1 &&
          float(tg.n - 1) >= 2.25f * ssp.locate_inv_h * (tg.wmax - tg.wmin);
 }
 
@@ -2204,7 +2402,7 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
     const FusedLaunch f{grid, s, g, *target, L.state, L.desc, L.chunk_off + n_band_keys,
                         items, axav, L.partial};
     const int w = fused_waves(nt, 4), wr = fused_waves(nt, 8);
-    if (fused_runs(*ssp, *target)) {
+    if (sparse_knots(*ssp, *target)) {
       if (wr <= 2) launch_fused<8, 2, 2>(f);
       else if (wr <= 4) launch_fused<8, 4, 2>(f);
       else if (wr <= 8) launch_fused<8, 8, 2>(f);
@@ -2257,15 +2455,17 @@ int cube_bwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   if (n == 0) return RBX_OK;
   const SspView g = view_of(*ssp);
   const int32_t nt = target->n;
-  const int n_tiles = (nt + kTile - 1) / kTile;
-  const int tps = (n_tiles + kBwdSlabs - 1) / kBwdSlabs;
+  // slabs of whole 64-bin groups, or of whole 256-bin blocks for the runs
+  const bool runs = sparse_knots(*ssp, *target);
+  const int unit = runs ? kBwdRunBins : kTile;
+  const int slab_bins = ((nt + unit - 1) / unit + kBwdSlabs - 1) / kBwdSlabs * unit;
   const int64_t items = int64_t(kBwdSlabs) * ((n + t.waves - 1) / t.waves);
   const int64_t grid = item_grid(items, t.persist, 64 * t.waves);
   switch (t.waves) {
-    case 1: launch_bwd<1>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, tps * kTile, axav, L.vpart, L.apart); break;
-    case 2: launch_bwd<2>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, tps * kTile, axav, L.vpart, L.apart); break;
-    case 8: launch_bwd<8>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, tps * kTile, axav, L.vpart, L.apart); break;
-    default: launch_bwd<4>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, tps * kTile, axav, L.vpart, L.apart);
+    case 1: launch_bwd<1>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
+    case 2: launch_bwd<2>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
+    case 8: launch_bwd<8>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
+    default: launch_bwd<4>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs);
   }
   if ((rc = check_launch(who))) return rc;
   hipLaunchKernelGGL(star_grad_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, g, *stars,
