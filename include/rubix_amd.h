@@ -337,6 +337,15 @@ int rbx_conv_axis_dot(const float* a, const float* b, int64_t n_outer,
                       int32_t n_taps, int32_t start, double* result,
                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* Taps of a normalised Gaussian g = exp(-x^2 / 2 sigma^2) / sum on the n
+ * positions x (rubix/telescope/psf/kernels.py:26-31,
+ * rubix/telescope/lsf/lsf.py:22-26): taps (float32), the same reversed, and
+ * dg/dsigma (double), evaluated in double.  sigma: one float32 on the device
+ * (sigma_f64 != 0: one double). */
+int rbx_gauss_taps(const double* x, int32_t n, const void* sigma,
+                   int32_t sigma_f64, float* taps, float* reversed,
+                   double* dtaps, void* stream);
+
 /* rbx_conv_axis_dot without a workspace argument and without allocating:
  * no counterpart in the reference; for callers that cannot allocate (code
  * under HIP graph capture, serving loops, harnesses that forbid hipMalloc).

@@ -132,6 +132,8 @@ SIGNATURES = {
                                  c_void_p, c_size_t, c_void_p]),
     "rbx_segment_cube_bwd": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int32, c_void_p,
                                      c_void_p]),
+    "rbx_gauss_taps": (c_int, [c_void_p, c_int32, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
+                               c_void_p]),
     "rbx_conv_axis": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int64, c_void_p, c_int32,
                               c_int32, c_void_p]),
     "rbx_psf_sep": (c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p,

@@ -76,20 +76,15 @@ def _xgrid(key, make, device):
 
 
 def _taps(key, make, sigma, device):
-    """(float32 taps, float64 d taps/d sigma) of the normalised Gaussian on the
-    grid `make()`.  A device-tensor sigma is evaluated on the device (no host
-    synchronisation); a python number on the host.  Both evaluate
-    g = exp(-x^2 / 2 sigma^2) / sum in float64 and round g once to float32."""
+    """(float32 taps, the taps reversed, float64 d taps/d sigma) of the
+    normalised Gaussian on the grid `make()`.  A device-tensor sigma is
+    evaluated on the device (one launch, no host synchronisation); a python
+    number on the host.  Both evaluate g = exp(-x^2 / 2 sigma^2) / sum in
+    float64 and round g once to float32."""
     if isinstance(sigma, torch.Tensor) and sigma.is_cuda:
-        x = _xgrid(key, make, device)
-        s = sigma.detach().to(device=device, dtype=torch.float64).reshape(())
-        e = torch.exp(-0.5 * x * x / (s * s))
-        g = e / e.sum()
-        x2 = x * x / (s * s * s)
-        dg = g * (x2 - (g * x2).sum())
-        return g.to(torch.float32), dg
+        return ops.gauss_taps(_xgrid(key, make, device), sigma.detach().to(device))
     g, dg = _norm_gauss(make(), float(sigma))
-    return _dev(g, device), _dev64(dg, device)
+    return _dev(g, device), _dev(g[::-1], device), _dev64(dg, device)
 
 
 def _dev(a, device):
@@ -138,25 +133,24 @@ class GaussianPSF(torch.autograd.Function):
     @staticmethod
     def forward(ctx, cube, sigma, size):
         ny, nx, nl = cube.shape
-        gt, dgt = _taps(("psf", size), lambda: psf_x(size), sigma, cube.device)
+        gt, grev, dgt = _taps(("psf", size), lambda: psf_x(size), sigma, cube.device)
         start = (size - 1) // 2
         cube = cube.contiguous()
         tmp = ops.conv_axis(cube, gt, ny, nx, nl, start)             # along x
         out = ops.conv_axis(tmp, gt, 1, ny, nx * nl, start)          # along y
         ctx.save_for_backward(cube, tmp)
-        ctx.taps = (gt, dgt)
+        ctx.taps = (grev, dgt)
         ctx.size = size
         return out
 
     @staticmethod
     def backward(ctx, gout):
         cube, tmp = ctx.saved_tensors
-        gt, dgt = ctx.taps
+        grev, dgt = ctx.taps
         m = ctx.size
         ny, nx, nl = cube.shape
         start = (m - 1) // 2
         rstart = m - 1 - start
-        grev = torch.flip(gt, (0,)).contiguous()
         gout = gout.contiguous()
         v = ops.conv_axis(gout, grev, 1, ny, nx * nl, rstart)        # Y^T
         gin = ops.conv_axis(v, grev, ny, nx, nl, rstart) if ctx.needs_input_grad[0] else None
@@ -179,26 +173,25 @@ class GaussianLSF(torch.autograd.Function):
         shape = cube.shape
         nl = shape[-1]
         ns = cube.numel() // nl
-        kt, dkt = _taps(("lsf", float(wave_res), factor), lambda: lsf_x(wave_res, factor), sigma,
+        kt, krev, dkt = _taps(("lsf", float(wave_res), factor), lambda: lsf_x(wave_res, factor), sigma,
                         cube.device)
         cube = cube.contiguous()
         out = ops.conv_axis(cube, kt, ns, nl, 1, factor)
         ctx.save_for_backward(cube)
-        ctx.taps = (kt, dkt)
+        ctx.taps = (krev, dkt)
         ctx.factor = factor
         return out
 
     @staticmethod
     def backward(ctx, gout):
         (cube,) = ctx.saved_tensors
-        kt, dkt = ctx.taps
-        L = kt.numel()
+        krev, dkt = ctx.taps
+        L = krev.numel()
         nl = cube.shape[-1]
         ns = cube.numel() // nl
         gout = gout.contiguous()
         gin = None
         if ctx.needs_input_grad[0]:
-            krev = torch.flip(kt, (0,)).contiguous()
             gin = ops.conv_axis(gout, krev, ns, nl, 1, L - 1 - ctx.factor)
         dsig = None
         if ctx.needs_input_grad[1]:
@@ -315,13 +308,13 @@ class BatchedPSF(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, cube, sigma, size, layout):
-        gt, dgt = _taps(("psf", size), lambda: psf_x(size), sigma, cube.device)
+        gt, grev, dgt = _taps(("psf", size), lambda: psf_x(size), sigma, cube.device)
         start = (size - 1) // 2
         cube = cube.contiguous()
         tmp = ops.conv_batch(cube, layout, 1, gt, start)   # along x
         out = ops.conv_batch(tmp, layout, 0, gt, start)    # along y
         ctx.save_for_backward(cube, tmp)
-        ctx.taps = (gt, dgt)
+        ctx.taps = (grev, dgt)
         ctx.size = size
         ctx.layout = layout
         return out
@@ -329,12 +322,11 @@ class BatchedPSF(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gout):
         cube, tmp = ctx.saved_tensors
-        gt, dgt = ctx.taps
+        grev, dgt = ctx.taps
         m = ctx.size
         layout = ctx.layout
         start = (m - 1) // 2
         rstart = m - 1 - start
-        grev = torch.flip(gt, (0,)).contiguous()
         gout = gout.contiguous()
         v = ops.conv_batch(gout, layout, 0, grev, rstart)
         gin = ops.conv_batch(v, layout, 1, grev, rstart) if ctx.needs_input_grad[0] else None

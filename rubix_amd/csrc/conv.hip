@@ -346,6 +346,45 @@ __global__ void __launch_bounds__(kDotThreads) dot_final_kernel(const double* __
   if (threadIdx.x == 0) *result = sm[0];
 }
 
+// ------------------------------------------------------------ Gaussian taps
+
+// Normalised Gaussian g = exp(-x^2 / 2 sigma^2) / sum on the grid x, its
+// reversed copy and dg/dsigma = g (x^2 / sigma^3 - sum_k g_k x_k^2 / sigma^3),
+// all in double (taps rounded once to float).  One workgroup, sums in a fixed
+// order.  As a dozen elementwise and reduction launches per PSF or LSF these
+// were a third of a 10 k-star step.
+template <class T>
+__global__ void __launch_bounds__(kDotThreads) gauss_taps_kernel(const double* __restrict__ x, int n,
+                                                                 const T* __restrict__ sigma,
+                                                                 float* __restrict__ taps,
+                                                                 float* __restrict__ reversed,
+                                                                 double* __restrict__ dtaps) {
+  __shared__ double sm[kDotThreads];
+  const double s = double(*sigma);
+  auto total = [&](double v) {
+    __syncthreads();
+    sm[threadIdx.x] = v;
+    __syncthreads();
+    for (int off = kDotThreads / 2; off > 0; off >>= 1) {
+      if (threadIdx.x < off) sm[threadIdx.x] += sm[threadIdx.x + off];
+      __syncthreads();
+    }
+    return sm[0];
+  };
+  auto bell = [&](int k) { return exp(-0.5 * x[k] * x[k] / (s * s)); };
+  double e = 0.0, ex = 0.0;
+  for (int k = threadIdx.x; k < n; k += kDotThreads) e += bell(k);
+  const double sum = total(e);
+  for (int k = threadIdx.x; k < n; k += kDotThreads) ex += bell(k) / sum * (x[k] * x[k] / (s * s * s));
+  const double mean = total(ex);
+  for (int k = threadIdx.x; k < n; k += kDotThreads) {
+    const double g = bell(k) / sum;
+    taps[k] = float(g);
+    reversed[n - 1 - k] = float(g);
+    dtaps[k] = g * (x[k] * x[k] / (s * s * s) - mean);
+  }
+}
+
 // ------------------------------------------------------------ batches
 //
 // A batch cube stacks the (nb, nb, n_lambda) cubes of several galaxies row
@@ -760,6 +799,21 @@ static int scratch_ptr(double** out, const char* who) {
 }  // namespace rbx
 
 extern "C" {
+
+int rbx_gauss_taps(const double* x, int32_t n, const void* sigma, int32_t sigma_f64, float* taps,
+                   float* reversed, double* dtaps, void* stream) {
+  using namespace rbx;
+  if (!x || !sigma || !taps || !reversed || !dtaps || n < 1)
+    return fail(RBX_EINVAL, "rbx_gauss_taps: bad arguments");
+  hipStream_t s = as_stream(stream);
+  if (sigma_f64)
+    hipLaunchKernelGGL(gauss_taps_kernel<double>, dim3(1), dim3(kDotThreads), 0, s, x, n,
+                       static_cast<const double*>(sigma), taps, reversed, dtaps);
+  else
+    hipLaunchKernelGGL(gauss_taps_kernel<float>, dim3(1), dim3(kDotThreads), 0, s, x, n,
+                       static_cast<const float*>(sigma), taps, reversed, dtaps);
+  return check_launch("rbx_gauss_taps");
+}
 
 int rbx_conv_axis(const float* in, float* out, int64_t n_outer, int32_t n_axis, int64_t n_inner,
                   const float* taps, int32_t n_taps, int32_t start, void* stream) {

@@ -351,6 +351,25 @@ def cube_backward(ssp: PreparedSSP, target: TargetGrid, ctx: CubeContext, dcube,
 
 # ---------------------------------------------------------------- convolutions
 
+def gauss_taps(x, sigma):
+    """Normalised Gaussian on the float64 grid x for a device-tensor sigma:
+    (float32 taps, the taps reversed, float64 d taps / d sigma)."""
+    _need_gpu(x, sigma)
+    if x.dtype != torch.float64:
+        raise TypeError("gauss_taps positions must be float64")
+    if sigma.numel() != 1:
+        raise ValueError(f"sigma must be one number, got shape {tuple(sigma.shape)}")
+    if sigma.dtype not in (torch.float32, torch.float64):
+        sigma = sigma.to(torch.float64)
+    x = x.contiguous()
+    n = x.numel()
+    taps = torch.empty(2, n, dtype=torch.float32, device=x.device)
+    dtaps = torch.empty(n, dtype=torch.float64, device=x.device)
+    call("rbx_gauss_taps", ptr(x), n, ptr(sigma), int(sigma.dtype == torch.float64), ptr(taps[0]),
+         ptr(taps[1]), ptr(dtaps), stream_handle(x.device))
+    return taps[0], taps[1], dtaps
+
+
 def conv_axis(x, taps, n_outer, n_axis, n_inner, start):
     """1D convolution along the middle axis of an (n_outer, n_axis, n_inner)
     view: out[o,x,i] = sum_t taps[t] * in[o, x + start - t, i] (zero pad)."""
