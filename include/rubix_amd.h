@@ -204,7 +204,8 @@ typedef struct rbx_galaxy {
 } rbx_galaxy;
 
 /* Launch tuning of the fused kernels (NULL = defaults): chunk = stars per
- * reduction chunk of the cube accumulation (16..65536, 0 = 256); waves =
+ * reduction chunk of the cube accumulation (16..65536, 0 = from the star and
+ * bin counts); waves =
  * wavefronts per workgroup of the per-star kernels (1, 2, 4, 8; 0 = 4);
  * persist = 0 for one workgroup per work item, k > 0 for persistent grids of
  * k workgroups per compute unit; flags: RBX_TUNE_TWO_PASS runs the forward

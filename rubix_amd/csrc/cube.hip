@@ -2149,7 +2149,7 @@ static int grid_for(int64_t n, int threads, int64_t cap = 1 << 20) {
 
 int tune_of(const rbx_tuning* t, Tune* out) {
   Tune d;
-  d.chunk = 256;
+  d.chunk = 0;
   d.waves = 4;
   d.persist = 0;
   d.flags = 0;
@@ -2159,7 +2159,7 @@ int tune_of(const rbx_tuning* t, Tune* out) {
     d.persist = t->persist;
     d.flags = t->flags;
   }
-  if (d.chunk < 16 || d.chunk > 65536)
+  if (d.chunk != 0 && (d.chunk < 16 || d.chunk > 65536))
     return fail(RBX_EINVAL, "rbx_tuning: chunk must be in [16, 65536] (0 = default)");
   if (d.waves != 1 && d.waves != 2 && d.waves != 4 && d.waves != 8)
     return fail(RBX_EINVAL, "rbx_tuning: waves must be 1, 2, 4 or 8 (0 = default)");
@@ -2310,7 +2310,7 @@ static int auto_chunk(int64_t n, int32_t nt) {
 size_t cube_workspace_impl(int64_t n, int32_t n_keys, int32_t nt, const Tune& t) {
   if (n < 0 || n_keys < 1 || nt < 1) return 0;
   SizeOnly so;
-  cube_layout(so, n, n_keys, nt, t.chunk, nullptr);
+  cube_layout(so, n, n_keys, nt, t.chunk ? t.chunk : auto_chunk(n, nt), nullptr);
   return so.s.used;
 }
 
@@ -2355,7 +2355,8 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   const int32_t nt = target->n;
   Carver c(workspace, workspace_bytes);
   CubeLayout L;
-  cube_layout(c, n, stars->n_keys, nt, t.chunk, &L);
+  const int chunk = t.chunk ? t.chunk : auto_chunk(n, nt);
+  cube_layout(c, n, stars->n_keys, nt, chunk, &L);
   if (!c.ok) return failf(RBX_EWORKSPACE, "%s: workspace too small", who);
   const SspView g = view_of(*ssp);
   const int32_t ns = stars->n_spaxel;
@@ -2393,7 +2394,7 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
     hipLaunchKernelGGL(star_sf_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, n, L.nn_part,
                        L.state);
   }
-  rc = build_chunks(L.offsets, n_band_keys, t.chunk, L.chunk_off, L.scan_blocks, L.desc, s);
+  rc = build_chunks(L.offsets, n_band_keys, chunk, L.chunk_off, L.scan_blocks, L.desc, s);
   if (rc) return rc;
   const int tpx = (n_tiles + 7) / 8;
   if (n > 0 && fused) {
@@ -2450,7 +2451,7 @@ int cube_bwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   const int64_t n = stars->n;
   Carver c(workspace, workspace_bytes);
   CubeLayout L;
-  cube_layout(c, n, stars->n_keys, target->n, t.chunk, &L, true);
+  cube_layout(c, n, stars->n_keys, target->n, 256, &L, true);  // no chunk arrays
   if (!c.ok) return failf(RBX_EWORKSPACE, "%s: workspace too small", who);
   if (n == 0) return RBX_OK;
   const SspView g = view_of(*ssp);
@@ -2495,7 +2496,6 @@ int rbx_ssp_prepare(const rbx_ssp* ssp, double* cum_out, int32_t* locate_out, vo
 size_t rbx_cube_workspace_size(int64_t n, int32_t n_keys, int32_t n_target) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
-  t.chunk = rbx::auto_chunk(n, n_target);
   return rbx::cube_workspace_impl(n, n_keys, n_target, t);
 }
 
@@ -2503,7 +2503,6 @@ int rbx_cube_fwd(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars* 
                  float* cube, void* workspace, size_t workspace_bytes, void* stream) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
-  if (stars && target) t.chunk = rbx::auto_chunk(stars->n, target->n);
   return rbx::cube_fwd_impl(ssp, target, stars, nullptr, t, cube, workspace, workspace_bytes,
                             rbx::as_stream(stream), "rbx_cube_fwd");
 }
@@ -2513,7 +2512,6 @@ int rbx_cube_fwd_ext(const rbx_ssp* ssp, const rbx_target* target, const rbx_sta
                      size_t workspace_bytes, void* stream) {
   rbx::Tune t;
   rbx::tune_of(nullptr, &t);
-  if (stars && target) t.chunk = rbx::auto_chunk(stars->n, target->n);
   return rbx::cube_fwd_impl(ssp, target, stars, ext, t, cube, workspace, workspace_bytes,
                             rbx::as_stream(stream), "rbx_cube_fwd_ext");
 }

@@ -8,7 +8,7 @@ namespace rbx {
 
 // Launch tuning resolved from rbx_tuning (NULL -> defaults).
 struct Tune {
-  int chunk;    // stars per reduction chunk of cube_accum
+  int chunk;    // stars per reduction chunk (0: from the star count)
   int waves;    // wavefronts per workgroup of star_norm / star_bwd
   int persist;  // 0 = one workgroup per work item, k = k workgroups per CU
   int flags;    // RBX_TUNE_TWO_PASS: no one-pass fused forward

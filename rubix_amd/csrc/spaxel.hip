@@ -27,7 +27,7 @@
 //   D-bit digits of the bucket index, each pass the same stable rank + scan +
 //   scatter over 2^D buckets, the scatter carrying each star's input index
 //   and bucket along; stable passes give the same order as the one-pass sort.
-//   Bucket offsets then come from a binary search of the sorted buckets.
+//   Bucket offsets then come from a binary search of the sorted stars.
 #include <math.h>
 #include <stdarg.h>
 #include <string.h>
@@ -234,23 +234,26 @@ static SortPlan make_plan(int64_t n, int32_t n_keys) {
 
 // Every star's rank in its tile, and for radix passes the input index and
 // bucket of every position: three n-element buffers (one index, two buckets)
-// beside the caller's perm.
+// beside the caller's perm.  The last radix pass writes no buckets, so with
+// two passes the ranks take the second bucket buffer.
 template <class S>
 static void sort_layout(S& c, const SortPlan& p, int32_t** table, int32_t** blocks,
                         uint16_t** rank, int32_t** tperm, int32_t** b0, int32_t** b1) {
   auto* t = c.template take<int32_t>(p.table);
   auto* bl = c.template take<int32_t>(p.nblk + 1);
-  auto* rk = c.template take<uint16_t>(p.n > 0 ? p.n : 1);
-  const int64_t rn = p.digit_bits ? (p.n > 0 ? p.n : 1) : 0;
+  const int64_t n1 = p.n > 0 ? p.n : 1;
+  const int64_t rn = p.digit_bits ? n1 : 0;
   auto* tp = c.template take<int32_t>(rn);
   auto* x0 = c.template take<int32_t>(rn);
   auto* x1 = c.template take<int32_t>(rn);
+  const bool shared = p.passes == 2;
+  auto* rk = c.template take<uint16_t>(shared ? 0 : n1);
   if (table) *table = reinterpret_cast<int32_t*>(t);
   if (blocks) *blocks = reinterpret_cast<int32_t*>(bl);
-  if (rank) *rank = reinterpret_cast<uint16_t*>(rk);
   if (tperm) *tperm = reinterpret_cast<int32_t*>(tp);
   if (b0) *b0 = reinterpret_cast<int32_t*>(x0);
   if (b1) *b1 = reinterpret_cast<int32_t*>(x1);
+  if (rank) *rank = shared ? reinterpret_cast<uint16_t*>(x1) : reinterpret_cast<uint16_t*>(rk);
 }
 
 struct SizerAdapter {
@@ -334,14 +337,16 @@ __global__ void __launch_bounds__(256) sort_scatter_kernel(
   }
 }
 
-// offsets[k] = number of sorted buckets below k, k in [0, n_keys].
-__global__ void bucket_offsets_kernel(const int32_t* __restrict__ bucket, int64_t n,
-                                      int32_t n_keys, int32_t* __restrict__ offsets) {
+// offsets[k] = number of sorted stars (perm) whose bucket lies below k, k in
+// [0, n_keys].
+__global__ void bucket_offsets_kernel(const int32_t* __restrict__ ids,
+                                      const int32_t* __restrict__ perm, int64_t n, int32_t n_keys,
+                                      int32_t* __restrict__ offsets) {
   for (int64_t k = gtid(); k <= n_keys; k += int64_t(gridDim.x) * blockDim.x) {
     int64_t lo = 0, hi = n;
     while (lo < hi) {
       const int64_t mid = (lo + hi) >> 1;
-      if (bucket[mid] < k) lo = mid + 1;
+      if (bucket_of(ids[perm[mid]], n_keys) < k) lo = mid + 1;
       else hi = mid;
     }
     offsets[k] = int32_t(lo);
@@ -444,7 +449,7 @@ int spaxel_sort_impl(const int32_t* ids, int64_t n, int32_t n_keys, int32_t* per
   for (int q = 0; q < p.passes; ++q) {
     const bool last = q == p.passes - 1;
     int32_t* pout = ((p.passes - 1 - q) & 1) ? tperm : perm;
-    int32_t* bout = bufs[q & 1];
+    int32_t* bout = last ? nullptr : bufs[q & 1];
     const int width = last ? p.nbits - q * p.digit_bits : p.digit_bits;
     int rc = sort_pass(p, in, q * p.digit_bits, mask, width, table, blocks, rank, src, ids,
                        pout, bout, last ? sorted : nullptr, nullptr, s);
@@ -453,7 +458,7 @@ int spaxel_sort_impl(const int32_t* ids, int64_t n, int32_t n_keys, int32_t* per
     src = pout;
   }
   hipLaunchKernelGGL(bucket_offsets_kernel, dim3(grid_for(int64_t(n_keys) + 1, 256)), dim3(256), 0,
-                     s, in, n, n_keys, offsets);
+                     s, ids, perm, n, n_keys, offsets);
   return check_launch("rbx_spaxel_sort");
 }
 
