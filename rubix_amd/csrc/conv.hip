@@ -9,19 +9,24 @@
 // convolution along the middle axis of an (n_outer, n_axis, n_inner) view.
 // Work is split so that index arithmetic happens once per workgroup item,
 // never per element (64-bit division per element would dominate):
-// * conv_tile_kernel (n_inner > 1 and an axis of at most kTileAxis, the
-//   spatial PSF passes): item = a block of 64 contiguous inner elements with
-//   the whole axis staged in LDS, so each input is read once.
+// * conv_cols_kernel (n_inner > 1 and one of the instantiated tap counts, the
+//   spatial PSF passes): a wavefront walks 64 contiguous inner elements along
+//   a segment of the axis with the last M inputs in registers, so each input
+//   is read once and a tap is one multiply-add, without LDS.
+// * conv_tile_kernel (other tap counts, an axis of at most kTileAxis): item =
+//   a block of 64 contiguous inner elements with the whole axis staged in LDS.
 // * conv_lines_kernel (n_inner > 1, longer axes): item = one (outer, axis)
 //   line and a chunk of up to kLineChunk contiguous inner elements; threads
 //   run along the contiguous inner axis.
 // * conv_rows_kernel (n_inner == 1, the LSF along lambda): item = a segment
-//   of kSeg outputs of one row; the segment's inputs plus the kernel's halo
-//   are staged in LDS once and every output reads its taps from LDS.
-// The batched PSF (rbx_conv_batch) uses row items of the batch cube: one
-// spaxel row and a chunk of lambda, its galaxy found once per item.  Every
-// output sums taps in the same order t = 0 .. m-1 as the flat definition.
+//   of at most kSeg outputs of one row; the segment's inputs plus the kernel's
+//   halo are staged in LDS once, a thread forms four consecutive outputs and
+//   reads 16 bytes of LDS per four taps.
+// The batched PSF (rbx_conv_batch) walks the lines of all galaxies as
+// conv_cols_kernel does.  Every output sums taps in the same order
+// t = 0 .. m-1 as the flat definition.
 #include <mutex>
+#include <type_traits>
 
 #include "rbx_common.h"
 
@@ -72,7 +77,7 @@ __global__ void conv2d_planes_kernel(const float* __restrict__ in, float* __rest
 constexpr int kDotThreads = 256;
 constexpr int kDotBlocksMax = 4096;
 constexpr int kLineChunk = 1024;  // inner elements per line item
-constexpr int kSeg = 2048;        // outputs per row item of the LSF
+constexpr int kSeg = 1024;        // most outputs per row item of the LSF
 constexpr int kHalo = 256;        // taps - 1 supported by the row kernel
 constexpr int kTileAxis = 240;    // longest axis the tiled line kernels stage (60 KB of LDS)
 
@@ -158,41 +163,177 @@ __global__ void __launch_bounds__(256) conv_tile_kernel(
   }
 }
 
-// Items: (row o, segment) of a row-contiguous convolution (n_inner == 1).
-// lds[k] = in[o, x0 + start - (m - 1) + k] (0 outside the row), so
-// out[o, x0 + v] = sum_t taps[t] lds[v + m - 1 - t].
+// One wavefront's lane of a convolution along a strided axis: outputs
+// x in [x0, x1) of the column at `src` (element xs at src + xs * stride, zero
+// outside [0, n)).  The last M inputs stay in registers (a ring whose places
+// are fixed by unrolling M steps), the next M are loaded ahead, and
+// sink(x, sum_t taps[t] in[x + start - t]) gets every output, its taps in the
+// order t = 0 .. M-1.  x0, x1 are wave-uniform; a lane without a column
+// (ok false) reads nothing.
+template <int M, class Acc, class Tap, class Sink>
+__device__ inline void column_walk(const float* __restrict__ src, int64_t stride, int n, bool ok,
+                                   int x0, int x1, int start, const Tap* __restrict__ taps,
+                                   Sink&& sink) {
+  Acc tap[M], ring[M];
+  float next[M];
+#pragma unroll
+  for (int t = 0; t < M; ++t) tap[t] = Acc(taps[t]);
+  auto load = [&](int xs) { return ok && xs >= 0 && xs < n ? src[int64_t(xs) * stride] : 0.f; };
+  // ring[u] holds the newest input x + start of step u (mod M)
+#pragma unroll
+  for (int u = 1; u < M; ++u) ring[u] = Acc(load(x0 + start - M + u));
+#pragma unroll
+  for (int u = 0; u < M; ++u) next[u] = load(x0 + start + u);
+  for (int xb = x0; xb < x1; xb += M) {
+    float cur[M];
+#pragma unroll
+    for (int u = 0; u < M; ++u) cur[u] = next[u];
+    if (xb + M < x1) {
+#pragma unroll
+      for (int u = 0; u < M; ++u) next[u] = load(xb + M + start + u);
+    }
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+      ring[u] = Acc(cur[u]);
+      if (xb + u < x1) {
+        Acc acc = Acc(0);
+#pragma unroll
+        for (int t = 0; t < M; ++t) acc += tap[t] * ring[(u - t + M) % M];
+        sink(xb + u, acc);
+      }
+    }
+  }
+}
+
+// Items, one per wavefront: (o, block of 64 contiguous inner elements,
+// segment of the axis), the segments of a block next to each other (they share
+// the halo in cache).  Bound by HBM: a 15-tap pass over 50 x 50 x 3721 (74 MB)
+// took 43 us from LDS and takes 19, an 11-tap pass over 300 x 300 x 1369
+// (0.99 GB, the axis too long for LDS) 1.3 ms and 0.25 (3.9 TB/s).
+template <int M>
+__global__ void __launch_bounds__(256) conv_cols_kernel(
+    const float* __restrict__ in, float* __restrict__ out, int n_axis, int64_t n_inner,
+    const float* __restrict__ taps, int start, int64_t n_blocks, int n_segs, int seg,
+    int64_t n_items) {
+  const int lane = threadIdx.x & 63;
+  const int64_t first = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t item = first; item < n_items; item += int64_t(gridDim.x) * 4) {
+    const int64_t blk = item / n_segs;
+    const int x0 = int(item - blk * n_segs) * seg;
+    const int x1 = x0 + seg < n_axis ? x0 + seg : n_axis;
+    const int64_t o = blk / n_blocks;
+    const int64_t i = (blk - o * n_blocks) * 64 + lane;
+    const bool ok = i < n_inner;
+    const int64_t base = o * n_axis * n_inner + (ok ? i : 0);
+    column_walk<M, float>(in + base, n_inner, n_axis, ok, x0, x1, start, taps,
+                          [&](int x, float v) {
+                            if (ok) out[base + int64_t(x) * n_inner] = v;
+                          });
+  }
+}
+
+// The taps of a row pass in LDS, reversed: tap[p] = taps[m - 1 - p].  (Read as
+// uniform global loads, each tap waited a scalar-cache round trip.)
+template <class Tap>
+__device__ inline void stage_taps(Tap* tap, const Tap* __restrict__ taps, int m) {
+  for (int p = threadIdx.x; p < m; p += blockDim.x) tap[p] = taps[m - 1 - p];
+}
+
+// Four consecutive outputs v .. v + 3 of a staged row: sum_t taps[t]
+// lds[v + e + m - 1 - t], the taps in the order t = 0 .. m-1 (tap[] from its
+// end), 16 bytes of LDS per four of them (v a multiple of 4; lds holds 4
+// floats past v + m + 2).
+template <class Acc, class Tap>
+__device__ inline void row_conv4(const float* lds, int v, const Tap* tap, int m, Acc (&acc)[4]) {
+  const float4* q4 = reinterpret_cast<const float4*>(lds + v);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = Acc(0);
+  int q = (m - 1) >> 2;
+  float4 hi = q4[q + 1];
+  float4 lo = q4[q];
+  auto window = [&](Acc (&w)[8]) {
+    w[0] = Acc(lo.x); w[1] = Acc(lo.y); w[2] = Acc(lo.z); w[3] = Acc(lo.w);
+    w[4] = Acc(hi.x); w[5] = Acc(hi.y); w[6] = Acc(hi.z); w[7] = Acc(hi.w);
+  };
+  {  // the last one to four places
+    Acc w[8];
+    window(w);
+#pragma unroll
+    for (int b = 3; b >= 0; --b) {
+      if (4 * q + b < m) {
+        const Acc tv = Acc(tap[4 * q + b]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += tv * w[b + e];
+      }
+    }
+  }
+  while (--q >= 0) {
+    hi = lo;
+    lo = q4[q];
+    Acc t4[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) t4[b] = Acc(tap[4 * q + b]);
+    Acc w[8];
+    window(w);
+#pragma unroll
+    for (int b = 3; b >= 0; --b) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += t4[b] * w[b + e];
+    }
+  }
+}
+
+// lds[k] = row[off + k] for k < len, 0 outside [0, n); 4 more zeros behind.
+__device__ inline void stage_row(float* lds, const float* __restrict__ row, int off, int len, int n) {
+  // every load in flight before the first is stored
+  constexpr int kLoads = (kSeg + kHalo + 4 + 255) / 256;
+  float v[kLoads];
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int k = threadIdx.x + 256 * u, xs = off + k;
+    v[u] = (k < len && xs >= 0 && xs < n) ? row[xs] : 0.f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int k = threadIdx.x + 256 * u;
+    if (k < len + 4) lds[k] = v[u];
+  }
+  __syncthreads();
+}
+
+// Four consecutive floats at any 4-byte alignment (one 16-byte access).
+struct alignas(4) Float4u {
+  float v[4];
+};
+
+// Items: (row o, segment of `seg` outputs, a multiple of 4 up to kSeg) of a
+// row-contiguous convolution (n_inner == 1).
+// lds[k] = in[o, x0 + start - (m - 1) + k] (0 outside the row: a tap past the
+// row's end adds taps[t] * 0), so out[o, x0 + v] = sum_t taps[t] lds[v + m - 1 - t].
+// 25 taps over 50 x 50 x 3721: 26 us with one LDS read per tap and output, 17
+// now (HBM: 14).
 __global__ void __launch_bounds__(256) conv_rows_kernel(
     const float* __restrict__ in, float* __restrict__ out, int n_axis,
-    const float* __restrict__ taps, int n_taps, int start, int64_t n_seg, int64_t n_items) {
-  __shared__ float lds[kSeg + kHalo];
+    const float* __restrict__ taps, int n_taps, int start, int64_t n_seg, int seg,
+    int64_t n_items) {
+  __shared__ __align__(16) float lds[kSeg + kHalo + 8];
+  __shared__ __align__(16) float tap[kHalo + 1];
+  stage_taps(tap, taps, n_taps);
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int64_t o = item / n_seg;
-    const int x0 = int(item - o * n_seg) * kSeg;
-    const float* row = in + o * n_axis;
-    const int off = x0 + start - (n_taps - 1);
-    const int len = kSeg + n_taps - 1;
-    __syncthreads();
-    for (int k = threadIdx.x; k < len; k += blockDim.x) {
-      const int xs = off + k;
-      lds[k] = (xs >= 0 && xs < n_axis) ? row[xs] : 0.f;
-    }
-    __syncthreads();
-    // lds is zero outside the row, so every tap reads it without a bounds
-    // test: a tap past the row's end adds taps[t] * 0
-    // outputs v, v + 256, v + 512, v + 768 of the thread as four independent
-    // sums (each in the order t = 0 .. m-1), hiding the LDS latency
-    for (int v0 = threadIdx.x; v0 < kSeg; v0 += 4 * 256) {
-      float acc[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int t = 0; t < n_taps; ++t) {
-        const float tv = taps[t];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) acc[k] += tv * lds[v0 + 256 * k + n_taps - 1 - t];
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int v = v0 + 256 * k;
-        if (v < kSeg && x0 + v < n_axis) out[o * n_axis + x0 + v] = acc[k];
-      }
+    const int x0 = int(item - o * n_seg) * seg;
+    const int len = n_axis - x0 < seg ? n_axis - x0 : seg;
+    stage_row(lds, in + o * n_axis, x0 + start - (n_taps - 1), (len + 3) / 4 * 4 + n_taps - 1, n_axis);
+    const int v = 4 * threadIdx.x;
+    if (v >= len) continue;
+    float acc[4];
+    row_conv4<float>(lds, v, tap, n_taps, acc);
+    float* dst = out + o * n_axis + x0 + v;
+    if (v + 4 <= len) {
+      *reinterpret_cast<Float4u*>(dst) = {{acc[0], acc[1], acc[2], acc[3]}};
+    } else {
+      for (int e = 0; v + e < len; ++e) dst[e] = e == 0 ? acc[0] : (e == 1 ? acc[1] : acc[2]);
     }
   }
 }
@@ -230,38 +371,59 @@ __global__ void __launch_bounds__(kDotThreads) conv_dot_lines_kernel(
   block_partial(acc, sm, partial);
 }
 
+// sum(a * conv(b)) per block over conv_cols_kernel's items, double taps.
+template <int M>
+__global__ void __launch_bounds__(kDotThreads) conv_dot_cols_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, int n_axis, int64_t n_inner,
+    const double* __restrict__ taps, int start, int64_t n_blocks, int n_segs, int seg,
+    int64_t n_items, double* __restrict__ partial) {
+  __shared__ double sm[kDotThreads];
+  double acc = 0.0;
+  const int lane = threadIdx.x & 63;
+  const int64_t first = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t item = first; item < n_items; item += int64_t(gridDim.x) * 4) {
+    const int64_t blk = item / n_segs;
+    const int x0 = int(item - blk * n_segs) * seg;
+    const int x1 = x0 + seg < n_axis ? x0 + seg : n_axis;
+    const int64_t o = blk / n_blocks;
+    const int64_t i = (blk - o * n_blocks) * 64 + lane;
+    const bool ok = i < n_inner;
+    const int64_t base = o * n_axis * n_inner + (ok ? i : 0);
+    column_walk<M, double>(b + base, n_inner, n_axis, ok, x0, x1, start, taps,
+                           [&](int x, double v) {
+                             if (ok) acc += double(a[base + int64_t(x) * n_inner]) * v;
+                           });
+  }
+  block_partial(acc, sm, partial);
+}
+
 // sum(a * conv(b)) per block, rows (n_inner == 1), double taps.
 __global__ void __launch_bounds__(kDotThreads) conv_dot_rows_kernel(
     const float* __restrict__ a, const float* __restrict__ b, int n_axis,
-    const double* __restrict__ taps, int n_taps, int start, int64_t n_seg, int64_t n_items,
-    double* __restrict__ partial) {
-  __shared__ float lds[kSeg + kHalo];
+    const double* __restrict__ taps, int n_taps, int start, int64_t n_seg, int seg,
+    int64_t n_items, double* __restrict__ partial) {
+  __shared__ __align__(16) float lds[kSeg + kHalo + 8];
+  __shared__ __align__(16) double tap[kHalo + 1];
   __shared__ double sm[kDotThreads];
   double acc = 0.0;
+  stage_taps(tap, taps, n_taps);
   for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int64_t o = item / n_seg;
-    const int x0 = int(item - o * n_seg) * kSeg;
-    const float* row = b + o * n_axis;
-    const int off = x0 + start - (n_taps - 1);
-    const int len = kSeg + n_taps - 1;
-    __syncthreads();
-    for (int k = threadIdx.x; k < len; k += blockDim.x) {
-      const int xs = off + k;
-      lds[k] = (xs >= 0 && xs < n_axis) ? row[xs] : 0.f;
-    }
-    __syncthreads();
-    for (int v0 = threadIdx.x; v0 < kSeg; v0 += 4 * 256) {
-      double c[4] = {0.0, 0.0, 0.0, 0.0};
-      for (int t = 0; t < n_taps; ++t) {
-        const double tv = taps[t];
+    const int x0 = int(item - o * n_seg) * seg;
+    const int len = n_axis - x0 < seg ? n_axis - x0 : seg;
+    stage_row(lds, b + o * n_axis, x0 + start - (n_taps - 1), (len + 3) / 4 * 4 + n_taps - 1, n_axis);
+    const int v = 4 * threadIdx.x;
+    if (v >= len) continue;
+    double c[4];
+    row_conv4<double>(lds, v, tap, n_taps, c);
+    const float* av = a + o * n_axis + x0 + v;
+    if (v + 4 <= len) {
+      const Float4u a4 = *reinterpret_cast<const Float4u*>(av);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) c[k] += tv * double(lds[v0 + 256 * k + n_taps - 1 - t]);
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int v = v0 + 256 * k;
-        if (v < kSeg && x0 + v < n_axis) acc += double(a[o * n_axis + x0 + v]) * c[k];
-      }
+      for (int e = 0; e < 4; ++e) acc += double(a4.v[e]) * c[e];
+    } else {
+      for (int e = 0; v + e < len; ++e)
+        acc += double(av[e]) * (e == 0 ? c[0] : (e == 1 ? c[1] : c[2]));
     }
   }
   block_partial(acc, sm, partial);
@@ -532,6 +694,20 @@ __device__ inline BatchLine batch_line(const rbx_galaxy* __restrict__ gal, const
   return b;
 }
 
+// A line that is the same for the whole wavefront, in scalar registers.
+__device__ inline BatchLine uniform_line(const BatchLine& b) {
+  auto scalar = [](int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(uint64_t(v) >> 32));
+    return int64_t(uint64_t(hi) << 32 | lo);
+  };
+  BatchLine u;
+  u.nb = __builtin_amdgcn_readfirstlane(b.nb);
+  u.base = scalar(b.base);
+  u.stride = scalar(b.stride);
+  return u;
+}
+
 // conv_batch_kernel's row item (row p, lambda chunk c) for tables that are
 // not packed.
 __device__ inline void batch_row_item(const float* __restrict__ in, float* __restrict__ out,
@@ -552,6 +728,33 @@ __device__ inline void batch_row_item(const float* __restrict__ in, float* __res
     }
     out[int64_t(p) * nt + l] = acc;
   }
+}
+
+// This thread's share of sum(a * conv(b)) over the row items of a table that is
+// not packed (rows of no galaxy add nothing).
+__device__ inline double batch_row_dots(const float* __restrict__ a, const float* __restrict__ bsrc,
+                                        const rbx_galaxy* __restrict__ gal, int n_gal, int n_rows,
+                                        int nt, int axis, const double* __restrict__ taps,
+                                        int n_taps, int start) {
+  double acc = 0.0;
+  const int n_chunks = (nt + kLineChunk - 1) / kLineChunk;
+  const int64_t n_items = int64_t(n_rows) * n_chunks;
+  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const int p = int(item / n_chunks);
+    const int l0 = int(item - int64_t(p) * n_chunks) * kLineChunk;
+    const int l1 = l0 + kLineChunk < nt ? l0 + kLineChunk : nt;
+    const BatchPos b = batch_pos(gal, n_gal, n_rows, nt, axis, int64_t(p) * nt);
+    if (!b.ok) continue;
+    for (int l = l0 + threadIdx.x; l < l1; l += blockDim.x) {
+      double c = 0.0;
+      for (int t = 0; t < n_taps; ++t) {
+        const int us = b.u + start - t;
+        if (us >= 0 && us < b.nb) c += taps[t] * double(bsrc[b.base + l + us * b.stride]);
+      }
+      acc += double(a[int64_t(p) * nt + l]) * c;
+    }
+  }
+  return acc;
 }
 
 __global__ void __launch_bounds__(256) conv_batch_tile_kernel(
@@ -607,6 +810,71 @@ __global__ void __launch_bounds__(256) conv_batch_tile_kernel(
   }
 }
 
+// conv_batch_tile_kernel for the instantiated tap counts: a wavefront walks
+// (line L, block of 64 lambda) as conv_cols_kernel does, lines of any length.
+template <int M>
+__global__ void __launch_bounds__(256) conv_batch_cols_kernel(
+    const float* __restrict__ in, float* __restrict__ out, const rbx_galaxy* __restrict__ gal,
+    int n_gal, int n_rows, int nt, int axis, const float* __restrict__ taps, int start) {
+  __shared__ int lines[kBatchGalMax + 1];
+  __shared__ int part[256];
+  const bool packed = batch_line_prefix(gal, n_gal, n_rows, lines, part);
+  if (!packed) {
+    const int n_chunks = (nt + kLineChunk - 1) / kLineChunk;
+    const int64_t n_items = int64_t(n_rows) * n_chunks;
+    for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x)
+      batch_row_item(in, out, gal, n_gal, n_rows, nt, axis, taps, M, start, n_chunks, item);
+    return;
+  }
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_lblk = (nt + 63) / 64;
+  const int64_t n_items = int64_t(lines[n_gal]) * n_lblk;
+  for (int64_t item = int64_t(blockIdx.x) * 4 + w; item < n_items; item += int64_t(gridDim.x) * 4) {
+    const int L = int(item / n_lblk);
+    const int l = int(item - int64_t(L) * n_lblk) * 64 + lane;
+    const bool ok = l < nt;
+    const BatchLine b = uniform_line(batch_line(gal, lines, n_gal, nt, axis, L));
+    const int64_t e0 = b.base + (ok ? l : 0);
+    column_walk<M, float>(in + e0, b.stride, b.nb, ok, 0, b.nb, start, taps,
+                          [&](int u, float v) {
+                            if (ok) out[e0 + u * b.stride] = v;
+                          });
+  }
+}
+
+// sum(a * conv(b)) per block over conv_batch_cols_kernel's items (packed
+// tables; the row items of conv_batch_dot_partial_kernel otherwise).
+template <int M>
+__global__ void __launch_bounds__(kDotThreads) conv_batch_dot_cols_kernel(
+    const float* __restrict__ a, const float* __restrict__ bsrc,
+    const rbx_galaxy* __restrict__ gal, int n_gal, int n_rows, int nt, int axis,
+    const double* __restrict__ taps, int start, double* __restrict__ partial) {
+  __shared__ int lines[kBatchGalMax + 1];
+  __shared__ int part[256];
+  __shared__ double sm[kDotThreads];
+  const bool packed = batch_line_prefix(gal, n_gal, n_rows, lines, part);
+  double acc = 0.0;
+  if (!packed) {
+    acc = batch_row_dots(a, bsrc, gal, n_gal, n_rows, nt, axis, taps, M, start);
+  } else {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_lblk = (nt + 63) / 64;
+    const int64_t n_items = int64_t(lines[n_gal]) * n_lblk;
+    for (int64_t item = int64_t(blockIdx.x) * 4 + w; item < n_items; item += int64_t(gridDim.x) * 4) {
+      const int L = int(item / n_lblk);
+      const int l = int(item - int64_t(L) * n_lblk) * 64 + lane;
+      const bool ok = l < nt;
+      const BatchLine b = uniform_line(batch_line(gal, lines, n_gal, nt, axis, L));
+      const int64_t e0 = b.base + (ok ? l : 0);
+      column_walk<M, double>(bsrc + e0, b.stride, b.nb, ok, 0, b.nb, start, taps,
+                             [&](int u, double v) {
+                               if (ok) acc += double(a[e0 + u * b.stride]) * v;
+                             });
+    }
+  }
+  block_partial(acc, sm, partial);
+}
+
 // sum(a * conv(b)) per block: line items of a packed table as
 // conv_batch_tile_kernel, else the row items of conv_batch_dot_partial_kernel.
 __global__ void __launch_bounds__(kDotThreads) conv_batch_dot_tile_kernel(
@@ -620,23 +888,7 @@ __global__ void __launch_bounds__(kDotThreads) conv_batch_dot_tile_kernel(
   const bool packed = batch_line_prefix(gal, n_gal, n_rows, lines, part);
   double acc = 0.0;
   if (!packed) {
-    const int n_chunks = (nt + kLineChunk - 1) / kLineChunk;
-    const int64_t n_items = int64_t(n_rows) * n_chunks;
-    for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-      const int p = int(item / n_chunks);
-      const int l0 = int(item - int64_t(p) * n_chunks) * kLineChunk;
-      const int l1 = l0 + kLineChunk < nt ? l0 + kLineChunk : nt;
-      const BatchPos b = batch_pos(gal, n_gal, n_rows, nt, axis, int64_t(p) * nt);
-      if (!b.ok) continue;
-      for (int l = l0 + threadIdx.x; l < l1; l += blockDim.x) {
-        double c = 0.0;
-        for (int t = 0; t < n_taps; ++t) {
-          const int us = b.u + start - t;
-          if (us >= 0 && us < b.nb) c += taps[t] * double(bsrc[b.base + l + us * b.stride]);
-        }
-        acc += double(a[int64_t(p) * nt + l]) * c;
-      }
-    }
+    acc = batch_row_dots(a, bsrc, gal, n_gal, n_rows, nt, axis, taps, n_taps, start);
   } else {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int n_lblk = (nt + 63) / 64;
@@ -714,15 +966,70 @@ static int dot_blocks(int64_t total) { return grid_for(total, kDotThreads * 8, k
 
 static int64_t item_blocks(int64_t items, int64_t cap) { return items < cap ? (items > 0 ? items : 1) : cap; }
 
+// Calls f with the tap count as a constant where conv_cols_kernel has it: the
+// odd sizes of a PSF kernel up to 25 pixels (M^2 multiply-adds of code and
+// about 3 M registers each).
+template <class F>
+static bool with_taps(int m, F&& f) {
+  switch (m) {
+    case 3: f(std::integral_constant<int, 3>{}); return true;
+    case 5: f(std::integral_constant<int, 5>{}); return true;
+    case 7: f(std::integral_constant<int, 7>{}); return true;
+    case 9: f(std::integral_constant<int, 9>{}); return true;
+    case 11: f(std::integral_constant<int, 11>{}); return true;
+    case 13: f(std::integral_constant<int, 13>{}); return true;
+    case 15: f(std::integral_constant<int, 15>{}); return true;
+    case 17: f(std::integral_constant<int, 17>{}); return true;
+    case 21: f(std::integral_constant<int, 21>{}); return true;
+    case 25: f(std::integral_constant<int, 25>{}); return true;
+    default: return false;
+  }
+}
+
+// conv_cols_kernel's items: segments of the axis so that about 16 000
+// wavefronts are there (two for each that fits the chip), but none shorter
+// than 16 outputs (its M - 1 halo inputs are read again, from cache).
+struct ColItems {
+  int64_t n_blocks, n_items;
+  int n_segs, seg;
+};
+
+static ColItems col_items(int64_t n_outer, int n_axis, int64_t n_inner) {
+  ColItems c;
+  c.n_blocks = (n_inner + 63) / 64;
+  const int64_t cols = n_outer * c.n_blocks;
+  int64_t want = (16384 + cols - 1) / cols;
+  const int64_t most = (n_axis + 15) / 16;
+  if (want > most) want = most;
+  c.seg = int((n_axis + want - 1) / want);
+  c.n_segs = (n_axis + c.seg - 1) / c.seg;
+  c.n_items = cols * c.n_segs;
+  return c;
+}
+
+// Outputs per row segment: the fewest segments of at most kSeg, of equal length.
+static int row_seg(int n_axis) {
+  const int n = (n_axis + kSeg - 1) / kSeg;
+  return ((n_axis + n - 1) / n + 3) / 4 * 4;
+}
+
 int conv_axis(const float* in, float* out, int64_t n_outer, int n_axis, int64_t n_inner,
               const float* taps, int n_taps, int start, hipStream_t s) {
   const int64_t total = n_outer * n_axis * n_inner;
   if (total == 0) return RBX_OK;
   if (n_inner == 1 && n_taps - 1 <= kHalo) {
-    const int64_t n_seg = (n_axis + kSeg - 1) / kSeg;
+    const int seg = row_seg(n_axis);
+    const int64_t n_seg = (n_axis + seg - 1) / seg;
     const int64_t items = n_outer * n_seg;
     hipLaunchKernelGGL(conv_rows_kernel, dim3(item_blocks(items, 1 << 20)), dim3(256), 0, s, in,
-                       out, n_axis, taps, n_taps, start, n_seg, items);
+                       out, n_axis, taps, n_taps, start, n_seg, seg, items);
+  } else if (n_inner > 1 && with_taps(n_taps, [&](auto m) {
+               const ColItems c = col_items(n_outer, n_axis, n_inner);
+               hipLaunchKernelGGL(conv_cols_kernel<decltype(m)::value>,
+                                  dim3(item_blocks((c.n_items + 3) / 4, 1 << 20)), dim3(256), 0, s,
+                                  in, out, n_axis, n_inner, taps, start, c.n_blocks, c.n_segs,
+                                  c.seg, c.n_items);
+             })) {
   } else if (n_inner > 1 && n_axis <= kTileAxis) {
     const int64_t n_blocks = (n_inner + 63) / 64;
     const int64_t items = n_outer * n_blocks;
@@ -748,9 +1055,16 @@ static int conv_axis_dot(const float* a, const float* b, int64_t n_outer, int n_
                          double* partial, int nblk, double* result, hipStream_t s,
                          const char* who) {
   if (n_inner == 1 && n_taps - 1 <= kHalo) {
-    const int64_t n_seg = (n_axis + kSeg - 1) / kSeg;
+    const int seg = row_seg(n_axis);
+    const int64_t n_seg = (n_axis + seg - 1) / seg;
     hipLaunchKernelGGL(conv_dot_rows_kernel, dim3(nblk), dim3(kDotThreads), 0, s, a, b, n_axis,
-                       taps, n_taps, start, n_seg, n_outer * n_seg, partial);
+                       taps, n_taps, start, n_seg, seg, n_outer * n_seg, partial);
+  } else if (n_inner > 1 && with_taps(n_taps, [&](auto m) {
+               const ColItems c = col_items(n_outer, n_axis, n_inner);
+               hipLaunchKernelGGL(conv_dot_cols_kernel<decltype(m)::value>, dim3(nblk),
+                                  dim3(kDotThreads), 0, s, a, b, n_axis, n_inner, taps, start,
+                                  c.n_blocks, c.n_segs, c.seg, c.n_items, partial);
+             })) {
   } else if (n_inner > 1 && n_axis <= kTileAxis) {
     const int64_t n_blocks = (n_inner + 63) / 64;
     hipLaunchKernelGGL(conv_dot_tile_kernel, dim3(nblk), dim3(kDotThreads),
@@ -901,6 +1215,12 @@ int rbx_conv_batch(const float* in, float* out, const rbx_galaxy* galaxies, int3
   if (total == 0) return RBX_OK;
   if (n_gal <= kBatchGalMax) {
     // persistent grid: every workgroup builds the table's line prefix once
+    if (with_taps(n_taps, [&](auto m) {
+          hipLaunchKernelGGL(conv_batch_cols_kernel<decltype(m)::value>, dim3(2048), dim3(256), 0,
+                             as_stream(stream), in, out, galaxies, n_gal, n_rows, n_target, axis,
+                             taps, start);
+        }))
+      return check_launch("rbx_conv_batch");
     hipLaunchKernelGGL(conv_batch_tile_kernel, dim3(2048), dim3(256),
                        size_t(kBatchTileAxis) * 64 * sizeof(float), as_stream(stream), in, out,
                        galaxies, n_gal, n_rows, n_target, axis, taps, n_taps, start);
@@ -928,7 +1248,12 @@ int rbx_conv_batch_dot(const float* a, const float* b, const rbx_galaxy* galaxie
     return fail(RBX_EWORKSPACE, "rbx_conv_batch_dot: workspace too small");
   hipStream_t s = as_stream(stream);
   double* partial = static_cast<double*>(workspace);
-  if (n_gal <= kBatchGalMax) {
+  if (n_gal <= kBatchGalMax && with_taps(n_taps, [&](auto m) {
+        hipLaunchKernelGGL(conv_batch_dot_cols_kernel<decltype(m)::value>, dim3(nblk),
+                           dim3(kDotThreads), 0, s, a, b, galaxies, n_gal, n_rows, n_target, axis,
+                           taps, start, partial);
+      })) {
+  } else if (n_gal <= kBatchGalMax) {
     hipLaunchKernelGGL(conv_batch_dot_tile_kernel, dim3(nblk), dim3(kDotThreads),
                        size_t(kBatchTileAxis) * 64 * sizeof(float), s, a, b, galaxies, n_gal,
                        n_rows, n_target, axis, taps, n_taps, start, partial);
