@@ -267,12 +267,17 @@ int rbx_ssp_lookup_bwd(const rbx_ssp* ssp, const float* met, const float* age, i
 
 /* scale_spectrum_by_mass (rubix/core/ifu.py:149-157): out[i, k] = in[i, k] *
  * scale[i] (out may alias in).  Its adjoint is the same call with the
- * incoming gradient, plus rbx_row_dot for d/dscale. */
+ * incoming gradient, plus rbx_row_dot for d/dscale (or rbx_scale_rows_bwd). */
 int rbx_scale_rows(const float* in, const float* scale, int64_t n, int32_t n_wave, float* out,
                    void* stream);
 /* out[i] = sum_k a[i, k] * b[i, k] (fixed-order reduction). */
 int rbx_row_dot(const float* a, const float* b, int64_t n, int32_t n_wave, float* out,
                 void* stream);
+/* Both adjoints of rbx_scale_rows in one pass over dout: din = dout * scale
+ * per row, dscale[i] = sum dout[i, :] in[i, :]. */
+int rbx_scale_rows_bwd(const float* dout, const float* scale, const float* in,
+                       int64_t n, int32_t nw, float* din, float* dscale,
+                       void* stream);
 
 /* doppler_shift_and_resampling (rubix/core/ifu.py:269-293 with
  * velocity_doppler_shift rubix/spectra/ifu.py:190 and resample_spectrum

@@ -123,6 +123,8 @@ SIGNATURES = {
                                    c_void_p, c_void_p]),
     "rbx_scale_rows": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
     "rbx_row_dot": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_void_p]),
+    "rbx_scale_rows_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p,
+                                   c_void_p, c_void_p]),
     "rbx_resample": (c_int, [POINTER(RbxSsp), POINTER(RbxTarget), c_void_p, c_void_p, c_int64,
                              c_int32, c_float, c_int64, c_void_p, c_void_p]),
     "rbx_resample_bwd": (c_int, [POINTER(RbxSsp), POINTER(RbxTarget), c_void_p, c_void_p, c_int64,

@@ -370,6 +370,9 @@ class ScaleByMass(torch.autograd.Function):
     def backward(ctx, dout):
         spectra, mass = ctx.saved_tensors
         dout = dout.contiguous()
+        if all(ctx.needs_input_grad[:2]):
+            ds, dm = ops.scale_rows_bwd(dout, mass, spectra)
+            return ds, dm.view_as(mass)
         ds = ops.scale_rows(dout, mass) if ctx.needs_input_grad[0] else None
         dm = ops.row_dot(dout, spectra).view_as(mass) if ctx.needs_input_grad[1] else None
         return ds, dm

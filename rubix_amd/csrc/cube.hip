@@ -178,117 +178,7 @@ __global__ void band_key_kernel(SspView g, rbx_stars st, int bands, int32_t* __r
   }
 }
 
-// ------------------------------------------------------------ segments
-//
-// The hot loops evaluate P_j = jnp.interp(target_j, w, S) with one lane per
-// target bin.  The segment starts from one probe of the locator table: the
-// cell of y = x / a gives k0 = (knots <= cell start) - 1 and the next knot,
-// and k = k0 + (next <= y).  That guess can be one knot off when x lies
-// within rounding distance of a knot, so it is then corrected with the exact
-// float32 predicate on the shifted knots w = fl(wave * a) that are loaded
-// anyway: step right while x >= w_r, left while x < w_l.  The result is
-// searchsorted(w, x, 'right') - 1 exactly, as the reference computes it
-// (the segment decides dP/da, which jumps at a knot).  The correction loop
-// also covers coarse tables (cells with several knots).
-
-// Element idx of an array with a wave-uniform base: the byte offset is formed
-// in 32 bits, so the load can use a scalar base plus a 32-bit vector offset
-// (every array read this way is below 4 GiB: checked by validate()).
-template <class T>
-__device__ inline T ld_at(const T* base, uint32_t idx) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + idx * uint32_t(sizeof(T)));
-}
-
-// Elements idx and idx + 1 in one 8-byte load (4-byte alignment is enough
-// for global memory on this target).
-struct alignas(4) Pair {
-  float lo, hi;
-};
-
-__device__ inline Pair ld_pair(const float* base, uint32_t idx) {
-  return *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(base) + idx * 4u);
-}
-
-// Elements idx .. idx + 3 in one 16-byte load (4-byte alignment, as above).
-struct alignas(4) Quad {
-  float v[4];
-};
-
-__device__ inline Quad ld_quad(const float* base, uint32_t idx) {
-  return *reinterpret_cast<const Quad*>(reinterpret_cast<const char*>(base) + idx * 4u);
-}
-
-// Per-star constants of the search: a, 1/a and the locator cell of target x
-// as x * c1 + c0.
-struct Shift {
-  float a, inv_a, c1, c0;
-};
-
-__device__ inline Shift shift_of(const SspView& g, float a, float inv_a) {
-  Shift h;
-  h.a = a;
-  h.inv_a = inv_a;
-  h.c1 = inv_a * g.loc_inv_h;
-  h.c0 = 1.0f - g.loc_x0 * g.loc_inv_h;
-  return h;
-}
-
-// jnp.interp segment [i0, i0 + 1] of target x: interpolation weight theta
-// (0 / 1 at the left / right clamp, 0 for a zero-width segment, as
-// jnp.interp's dx == 0 branch) and, for the adjoint, kappa = lambda(x) /
-// (w_r - w_l) with lambda(x) = l0 + theta (l1 - l0) on the unshifted knots,
-// so that dP/da = -kappa (S1 - S0) inside the grid (0 at the clamps).
-struct Knots {
-  uint32_t i0;
-  float theta;
-  float kappa;
-};
-
-template <bool kKappa>
-__device__ inline Knots knots_of(const SspView& g, float x, const Shift& h) {
-  const int n = g.n_wave;
-  float fm = fmaf(x, h.c1, h.c0);
-  fm = fminf(fmaxf(fm, 0.f), float(g.n_loc - 1));
-  const int4 e = ld_at(reinterpret_cast<const int4*>(g.loc), uint32_t(fm));
-  const float y = x * h.inv_a;
-  const float e1 = __int_as_float(e.y), e2 = __int_as_float(e.z), e3 = __int_as_float(e.w);
-  const int k = e.x + (e2 <= y ? 1 : 0);  // e2 = the knot after k0 (see ssp_locate_kernel)
-  int i = k + 1 < 1 ? 1 : (k + 1 > n - 1 ? n - 1 : k + 1);
-  // the segment's knots from the entry: i - 1 - b is 0 or 1
-  const int b = e.x < n - 2 ? e.x : n - 2;
-  const bool hi = (i - 1 - b) > 0;
-  Pair lp;
-  lp.lo = hi ? e2 : e1;
-  lp.hi = hi ? e3 : e2;
-  float wl = mul_nocontract(lp.lo, h.a), wr = mul_nocontract(lp.hi, h.a);
-  // exact segment: i in [1, n-1] moves monotonically, so the loop ends.
-  // Corrections are rare; a wave vote keeps the common case to one
-  // compare and a uniform branch.
-  bool step = (x >= wr && i < n - 1) || (x < wl && i > 1);
-  if (__ballot(step)) {
-    while (step) {
-      i += x >= wr ? 1 : -1;
-      lp = ld_pair(g.wave, uint32_t(i - 1));
-      wl = mul_nocontract(lp.lo, h.a);
-      wr = mul_nocontract(lp.hi, h.a);
-      step = (x >= wr && i < n - 1) || (x < wl && i > 1);
-    }
-  }
-  const uint32_t i0 = uint32_t(i - 1);
-  const float l0 = lp.lo, l1 = lp.hi;
-  const float dx = wr - wl;
-  const float r = __builtin_amdgcn_rcpf(dx);
-  const bool flat = !(dx > 0.f);
-  const float th = flat ? 0.f : (x - wl) * r;
-  const bool left = (i == 1) && (x < wl);
-  const bool right = (i == n - 1) && (x > wr);
-  Knots K;
-  K.i0 = i0;
-  K.theta = left ? 0.f : (right ? 1.f : th);
-  K.kappa = 0.f;
-  if (kKappa) K.kappa = (left || right || flat) ? 0.f : (l0 + th * (l1 - l0)) * r;
-  return K;
-}
+// ------------------------------------------------------------ rows
 
 // Row pointers of a star's four template corners (uniform over the wave).
 struct Rows {

@@ -98,26 +98,138 @@ __device__ inline int locate(const SspView& g, float x, float a, float inv_a) {
   return k;
 }
 
-// jnp.interp bookkeeping for one target x: segment [i-1, i] with
-// i = clip(k+1, 1, n-1), theta = (x - w[i-1]) / (w[i] - w[i-1]), and the
-// clamp side (-1: x < w[0] -> S[0]; +1: x > w[n-1] -> S[n-1]; 0 interior).
-struct Seg {
-  int i;
-  int side;
-  float theta;
-  float wl, wr;
+// ------------------------------------------------------------ segments
+//
+// The fused and the resampling kernels evaluate P_j = jnp.interp(target_j, w, S)
+// with one lane per target bin.  The segment starts from one probe of the locator table: the
+// cell of y = x / a gives k0 = (knots <= cell start) - 1 and the next knot,
+// and k = k0 + (next <= y).  That guess can be one knot off when x lies
+// within rounding distance of a knot, so it is then corrected with the exact
+// float32 predicate on the shifted knots w = fl(wave * a) that are loaded
+// anyway: step right while x >= w_r, left while x < w_l.  The result is
+// searchsorted(w, x, 'right') - 1 exactly, as the reference computes it
+// (the segment decides dP/da, which jumps at a knot).  The correction loop
+// also covers coarse tables (cells with several knots).
+
+// Element idx of an array with a wave-uniform base: the byte offset is formed
+// in 32 bits, so the load can use a scalar base plus a 32-bit vector offset
+// (every array read this way is below 4 GiB: checked by validate()).
+template <class T>
+__device__ inline T ld_at(const T* base, uint32_t idx) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + idx * uint32_t(sizeof(T)));
+}
+
+// Elements idx and idx + 1 in one 8-byte load (4-byte alignment is enough
+// for global memory on this target).
+struct alignas(4) Pair {
+  float lo, hi;
 };
 
-__device__ inline Seg segment(const SspView& g, float x, float a, float inv_a) {
-  const int k = locate(g, x, a, inv_a);
+__device__ inline Pair ld_pair(const float* base, uint32_t idx) {
+  return *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(base) + idx * 4u);
+}
+
+// Elements idx .. idx + 3 in one 16-byte load (4-byte alignment, as above).
+struct alignas(4) Quad {
+  float v[4];
+};
+
+__device__ inline Quad ld_quad(const float* base, uint32_t idx) {
+  return *reinterpret_cast<const Quad*>(reinterpret_cast<const char*>(base) + idx * 4u);
+}
+
+// Per-star constants of the search: a, 1/a and the locator cell of target x
+// as x * c1 + c0.
+struct Shift {
+  float a, inv_a, c1, c0;
+};
+
+__device__ inline Shift shift_of(const SspView& g, float a, float inv_a) {
+  Shift h;
+  h.a = a;
+  h.inv_a = inv_a;
+  h.c1 = inv_a * g.loc_inv_h;
+  h.c0 = 1.0f - g.loc_x0 * g.loc_inv_h;
+  return h;
+}
+
+// jnp.interp segment [i0, i0 + 1] of target x: interpolation weight theta
+// (0 / 1 at the left / right clamp, 0 for a zero-width segment, as
+// jnp.interp's dx == 0 branch) and, for the adjoint, kappa = lambda(x) /
+// (w_r - w_l) with lambda(x) = l0 + theta (l1 - l0) on the unshifted knots,
+// so that dP/da = -kappa (S1 - S0) inside the grid (0 at the clamps).
+struct Knots {
+  uint32_t i0;
+  float theta;
+  float kappa;
+};
+
+// The segments of U targets, their locator probes in flight together.
+template <int U, bool kKappa>
+__device__ inline void knots_group(const SspView& g, const float (&x)[U], const Shift& h,
+                                   Knots (&K)[U]) {
   const int n = g.n_wave;
-  Seg s;
-  s.i = k + 1 < 1 ? 1 : (k + 1 > n - 1 ? n - 1 : k + 1);
-  s.wl = knot(g, s.i - 1, a);
-  s.wr = knot(g, s.i, a);
-  s.side = (k < 0) ? -1 : ((k >= n - 1 && x > s.wr) ? 1 : 0);
-  s.theta = (x - s.wl) / (s.wr - s.wl);
-  return s;
+  int4 e[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float fm = fminf(fmaxf(fmaf(x[u], h.c1, h.c0), 0.f), float(g.n_loc - 1));
+    e[u] = ld_at(reinterpret_cast<const int4*>(g.loc), uint32_t(fm));
+  }
+  int i[U];
+  Pair lp[U];
+  float wl[U], wr[U];
+  bool any = false;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float y = x[u] * h.inv_a;
+    const float e1 = __int_as_float(e[u].y), e2 = __int_as_float(e[u].z), e3 = __int_as_float(e[u].w);
+    const int k = e[u].x + (e2 <= y ? 1 : 0);  // e2 = the knot after k0 (see ssp_locate_kernel)
+    i[u] = k + 1 < 1 ? 1 : (k + 1 > n - 1 ? n - 1 : k + 1);
+    // the segment's knots from the entry: i - 1 - b is 0 or 1
+    const int b = e[u].x < n - 2 ? e[u].x : n - 2;
+    const bool hi = (i[u] - 1 - b) > 0;
+    lp[u].lo = hi ? e2 : e1;
+    lp[u].hi = hi ? e3 : e2;
+    wl[u] = mul_nocontract(lp[u].lo, h.a);
+    wr[u] = mul_nocontract(lp[u].hi, h.a);
+    any |= (x[u] >= wr[u] && i[u] < n - 1) || (x[u] < wl[u] && i[u] > 1);
+  }
+  // exact segment: i in [1, n-1] moves monotonically, so the loop ends.
+  // Corrections are rare; a wave vote keeps the common case to one
+  // compare and a uniform branch.
+  if (__ballot(any)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      while ((x[u] >= wr[u] && i[u] < n - 1) || (x[u] < wl[u] && i[u] > 1)) {
+        i[u] += x[u] >= wr[u] ? 1 : -1;
+        lp[u] = ld_pair(g.wave, uint32_t(i[u] - 1));
+        wl[u] = mul_nocontract(lp[u].lo, h.a);
+        wr[u] = mul_nocontract(lp[u].hi, h.a);
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float dx = wr[u] - wl[u];
+    const float r = __builtin_amdgcn_rcpf(dx);
+    const bool flat = !(dx > 0.f);
+    const float th = flat ? 0.f : (x[u] - wl[u]) * r;
+    const bool left = (i[u] == 1) && (x[u] < wl[u]);
+    const bool right = (i[u] == n - 1) && (x[u] > wr[u]);
+    K[u].i0 = uint32_t(i[u] - 1);
+    K[u].theta = left ? 0.f : (right ? 1.f : th);
+    K[u].kappa = 0.f;
+    if (kKappa)
+      K[u].kappa = (left || right || flat) ? 0.f : (lp[u].lo + th * (lp[u].hi - lp[u].lo)) * r;
+  }
+}
+
+template <bool kKappa>
+__device__ inline Knots knots_of(const SspView& g, float x, const Shift& h) {
+  Knots K[1];
+  const float xs[1] = {x};
+  knots_group<1, kKappa>(g, xs, h, K);
+  return K[0];
 }
 
 // Bilinear cell of one star (interp2d linear): corner weights, their

@@ -601,6 +601,23 @@ def row_dot(a, b):
     return out
 
 
+def scale_rows_bwd(dout, scale, x):
+    """Both adjoints of scale_rows in one pass: (dout[i, :] * scale[i],
+    sum dout[i, :] x[i, :])."""
+    _need_gpu(dout, scale, x)
+    dout = _rows(dout, "dout")
+    x = _rows(x, "spectra")
+    scale = _f32(scale, "mass").reshape(-1)
+    if dout.shape != x.shape or scale.numel() != x.shape[0]:
+        raise ValueError(f"scale_rows_bwd: dout {tuple(dout.shape)}, spectra {tuple(x.shape)}, "
+                         f"{scale.numel()} scales")
+    dx = torch.empty_like(x)
+    dscale = torch.empty(x.shape[0], dtype=torch.float32, device=x.device)
+    call("rbx_scale_rows_bwd", ptr(dout), ptr(scale), ptr(x), x.shape[0], x.shape[1], ptr(dx),
+         ptr(dscale), stream_handle(x.device))
+    return dx, dscale
+
+
 def resample(ssp: PreparedSSP, target: TargetGrid, spectra, velocity, vel_comp=2,
              c=SPEED_OF_LIGHT):
     """doppler_shift_and_resampling on materialised spectra (N, n_wave)."""
