@@ -998,7 +998,7 @@ static ColItems col_items(int64_t n_outer, int n_axis, int64_t n_inner) {
   ColItems c;
   c.n_blocks = (n_inner + 63) / 64;
   const int64_t cols = n_outer * c.n_blocks;
-  int64_t want = (16384 + cols - 1) / cols;
+  int64_t want = cols > 0 ? (16384 + cols - 1) / cols : 1;
   const int64_t most = (n_axis + 15) / 16;
   if (want > most) want = most;
   c.seg = int((n_axis + want - 1) / want);
