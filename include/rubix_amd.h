@@ -251,6 +251,14 @@ int rbx_conv_batch_dot(const float* a, const float* b, const rbx_galaxy* galaxie
                        const double* taps, int32_t n_taps, int32_t start,
                        double* out, void* workspace, size_t workspace_bytes,
                        void* stream);
+/* rbx_conv_axis_bwd for one pass over every galaxy of a batch cube. */
+int rbx_conv_batch_bwd(const float* dout, const float* in, float* din,
+                       const rbx_galaxy* galaxies, int32_t n_gal,
+                       int32_t n_rows, int32_t n_target, int32_t axis,
+                       const float* reversed, const double* dtaps,
+                       int32_t n_taps, int32_t start, const double* add,
+                       double* result, float* result32, void* workspace,
+                       size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------- per step
  * One kernel per rubix.core step, materialising the same per-star arrays the
@@ -351,6 +359,20 @@ int rbx_conv_axis_dot(const float* a, const float* b, int64_t n_outer,
 int rbx_gauss_taps(const double* x, int32_t n, const void* sigma,
                    int32_t sigma_f64, float* taps, float* reversed,
                    double* dtaps, void* stream);
+
+/* The adjoint of rbx_conv_axis and the derivative in a parameter of its taps
+ * together: din = the convolution of dout with the reversed taps from
+ * n_taps - 1 - start, result[0] = (add ? add[0] : 0) + sum dout * conv(in) with
+ * the double derivative taps dtaps from `start` (result32, nullable: the same in
+ * float32).  One pass over dout and in for the LSF and for centred kernels of
+ * odd size up to 15, else as the two calls.  workspace: rbx_dot_workspace_size
+ * of the element count. */
+int rbx_conv_axis_bwd(const float* dout, const float* in, float* din,
+                      int64_t n_outer, int32_t n_axis, int64_t n_inner,
+                      const float* reversed, const double* dtaps,
+                      int32_t n_taps, int32_t start, const double* add,
+                      double* result, float* result32, void* workspace,
+                      size_t workspace_bytes, void* stream);
 
 /* rbx_conv_axis_dot without a workspace argument and without allocating:
  * no counterpart in the reference; for callers that cannot allocate (code

@@ -93,6 +93,9 @@ SIGNATURES = {
     "rbx_conv_batch_dot": (c_int, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                    c_int32, c_void_p, c_int32, c_int32, c_void_p, c_void_p,
                                    c_size_t, c_void_p]),
+    "rbx_conv_batch_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
+                                   c_int32, c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p,
+                                   c_void_p, c_void_p, c_size_t, c_void_p]),
     "rbx_filter_particles": (c_int, [c_void_p, c_int64, c_int64, c_float, c_float, c_void_p,
                                      c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                      c_void_p]),
@@ -145,6 +148,9 @@ SIGNATURES = {
     "rbx_dot_workspace_size": (c_size_t, [c_int64]),
     "rbx_conv_axis_dot": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int64, c_void_p, c_int32,
                                   c_int32, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "rbx_conv_axis_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int64, c_void_p,
+                                  c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p,
+                                  c_size_t, c_void_p]),
     "rbx_conv_axis_dot_noalloc": (c_int, [c_void_p, c_void_p, c_int64, c_int32, c_int64, c_void_p,
                                           c_int32, c_int32, c_void_p, c_void_p]),
 }

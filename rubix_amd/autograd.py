@@ -152,6 +152,11 @@ class GaussianPSF(torch.autograd.Function):
         start = (m - 1) // 2
         rstart = m - 1 - start
         gout = gout.contiguous()
+        if all(ctx.needs_input_grad[:2]):
+            # <G, Y' X C> with v = Y^T G, then <v, X' C> with X^T v
+            v, d1, _ = ops.conv_axis_bwd(gout, tmp, grev, dgt, 1, ny, nx * nl, start)
+            gin, _, dsig = ops.conv_axis_bwd(v, cube, grev, dgt, ny, nx, nl, start, add=d1)
+            return gin, dsig, None
         v = ops.conv_axis(gout, grev, 1, ny, nx * nl, rstart)        # Y^T
         gin = ops.conv_axis(v, grev, ny, nx, nl, rstart) if ctx.needs_input_grad[0] else None
         dsig = None
@@ -190,6 +195,9 @@ class GaussianLSF(torch.autograd.Function):
         nl = cube.shape[-1]
         ns = cube.numel() // nl
         gout = gout.contiguous()
+        if all(ctx.needs_input_grad[:2]):
+            gin, _, dsig = ops.conv_axis_bwd(gout, cube, krev, dkt, ns, nl, 1, ctx.factor)
+            return gin, dsig, None, None
         gin = None
         if ctx.needs_input_grad[0]:
             gin = ops.conv_axis(gout, krev, ns, nl, 1, L - 1 - ctx.factor)
@@ -328,6 +336,10 @@ class BatchedPSF(torch.autograd.Function):
         start = (m - 1) // 2
         rstart = m - 1 - start
         gout = gout.contiguous()
+        if all(ctx.needs_input_grad[:2]):
+            v, d1, _ = ops.conv_batch_bwd(gout, tmp, layout, 0, grev, dgt, start)
+            gin, _, dsig = ops.conv_batch_bwd(v, cube, layout, 1, grev, dgt, start, add=d1)
+            return gin, dsig, None, None
         v = ops.conv_batch(gout, layout, 0, grev, rstart)
         gin = ops.conv_batch(v, layout, 1, grev, rstart) if ctx.needs_input_grad[0] else None
         dsig = None

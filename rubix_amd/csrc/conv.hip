@@ -205,6 +205,66 @@ __device__ inline void column_walk(const float* __restrict__ src, int64_t stride
   }
 }
 
+// The adjoint's walk for a centred kernel (start = (M - 1) / 2, M odd) along
+// the column of a (the incoming gradient) and b (the forward's input) at once:
+// emit(x, sum_t rev[t] a[x + start - t]) is the transposed convolution, and
+// the sum of a[x] sum_t dtaps[t] b[x + start - t] (double) is returned; a[x] is in
+// the ring.  a and b are read once for both.
+template <int M, class Emit>
+__device__ inline double column_walk_bwd(const float* __restrict__ a, const float* __restrict__ b,
+                                         int64_t stride, int n, bool ok, int x0, int x1,
+                                         const float* __restrict__ rev,
+                                         const double* __restrict__ dtaps, Emit&& emit) {
+  constexpr int start = (M - 1) / 2;
+  float ring[M], next_a[M], next_b[M];
+  double ringd[M];
+  double dot = 0.0;
+  auto inside = [&](int xs) { return ok && xs >= 0 && xs < n; };
+  auto load = [&](const float* src, int xs) { return inside(xs) ? src[int64_t(xs) * stride] : 0.f; };
+#pragma unroll
+  for (int u = 1; u < M; ++u) {
+    ring[u] = load(a, x0 + start - M + u);
+    ringd[u] = double(load(b, x0 + start - M + u));
+  }
+#pragma unroll
+  for (int u = 0; u < M; ++u) {
+    next_a[u] = load(a, x0 + start + u);
+    next_b[u] = load(b, x0 + start + u);
+  }
+  for (int xb = x0; xb < x1; xb += M) {
+    float cur_a[M], cur_b[M];
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+      cur_a[u] = next_a[u];
+      cur_b[u] = next_b[u];
+    }
+    if (xb + M < x1) {
+#pragma unroll
+      for (int u = 0; u < M; ++u) {
+        next_a[u] = load(a, xb + M + start + u);
+        next_b[u] = load(b, xb + M + start + u);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < M; ++u) {
+      ring[u] = cur_a[u];
+      ringd[u] = double(cur_b[u]);
+      if (xb + u < x1) {
+        float acc = 0.f;
+        double c = 0.0;
+#pragma unroll
+        for (int t = 0; t < M; ++t) {
+          acc += rev[t] * ring[(u - t + M) % M];
+          c += dtaps[t] * ringd[(u - t + M) % M];
+        }
+        emit(xb + u, acc);
+        dot += double(ring[(u - start + M) % M]) * c;
+      }
+    }
+  }
+  return ok ? dot : 0.0;
+}
+
 // Items, one per wavefront: (o, block of 64 contiguous inner elements,
 // segment of the axis), the segments of a block next to each other (they share
 // the halo in cache).  Bound by HBM: a 15-tap pass over 50 x 50 x 3721 (74 MB)
@@ -283,22 +343,30 @@ __device__ inline void row_conv4(const float* lds, int v, const Tap* tap, int m,
   }
 }
 
-// lds[k] = row[off + k] for k < len, 0 outside [0, n); 4 more zeros behind.
-__device__ inline void stage_row(float* lds, const float* __restrict__ row, int off, int len, int n) {
-  // every load in flight before the first is stored
-  constexpr int kLoads = (kSeg + kHalo + 4 + 255) / 256;
-  float v[kLoads];
+// A staged row segment of the LDS buffers below: a thread's share of
+// row[off + k], k < len, 0 outside [0, n), and 4 more zeros behind.
+constexpr int kRowLoads = (kSeg + kHalo + 4 + 255) / 256;
+__device__ inline void load_row(float* v, const float* __restrict__ row, int off, int len, int n) {
 #pragma unroll
-  for (int u = 0; u < kLoads; ++u) {
+  for (int u = 0; u < kRowLoads; ++u) {
     const int k = threadIdx.x + 256 * u, xs = off + k;
     v[u] = (k < len && xs >= 0 && xs < n) ? row[xs] : 0.f;
   }
-  __syncthreads();
+}
+__device__ inline void store_row(float* lds, const float* v, int len) {
 #pragma unroll
-  for (int u = 0; u < kLoads; ++u) {
+  for (int u = 0; u < kRowLoads; ++u) {
     const int k = threadIdx.x + 256 * u;
     if (k < len + 4) lds[k] = v[u];
   }
+}
+
+// lds[k] = row[off + k] for k < len, 0 outside [0, n); 4 more zeros behind.
+__device__ inline void stage_row(float* lds, const float* __restrict__ row, int off, int len, int n) {
+  float v[kRowLoads];  // every load in flight before the first is stored
+  load_row(v, row, off, len, n);
+  __syncthreads();
+  store_row(lds, v, len);
   __syncthreads();
 }
 
@@ -429,6 +497,104 @@ __global__ void __launch_bounds__(kDotThreads) conv_dot_rows_kernel(
   block_partial(acc, sm, partial);
 }
 
+// conv_cols_kernel and conv_dot_cols_kernel of the adjoint in one pass over a
+// and b.  Bound by HBM: two cubes read and one written, where the two passes
+// read three.  300 x 300 x 1369, 11 taps: 397 us, 490 for the two.  Up to 15 taps:
+// the two rings take 8 registers per tap, and past 128 of them fewer waves are
+// resident than the loads need.
+template <int M>
+__global__ void __launch_bounds__(kDotThreads) conv_bwd_cols_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out, int n_axis,
+    int64_t n_inner, const float* __restrict__ rev, const double* __restrict__ dtaps,
+    int64_t n_blocks, int n_segs, int seg, int64_t n_items, double* __restrict__ partial) {
+  __shared__ double sm[kDotThreads];
+  double acc = 0.0;
+  const int lane = threadIdx.x & 63;
+  const int64_t first = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t item = first; item < n_items; item += int64_t(gridDim.x) * 4) {
+    const int64_t blk = item / n_segs;
+    const int x0 = int(item - blk * n_segs) * seg;
+    const int x1 = x0 + seg < n_axis ? x0 + seg : n_axis;
+    const int64_t o = blk / n_blocks;
+    const int64_t i = (blk - o * n_blocks) * 64 + lane;
+    const bool ok = i < n_inner;
+    const int64_t base = o * n_axis * n_inner + (ok ? i : 0);
+    acc += column_walk_bwd<M>(a + base, b + base, n_inner, n_axis, ok, x0, x1, rev, dtaps,
+                              [&](int x, float v) {
+                                if (ok) out[base + int64_t(x) * n_inner] = v;
+                              });
+  }
+  block_partial(acc, sm, partial);
+}
+
+// conv_rows_kernel and conv_dot_rows_kernel of the adjoint in one pass:
+// out = conv(a, rev) from rstart = m - 1 - start, and sum(a * conv(b, dtaps)).
+// The workgroup's LDS holds one item, so the next one's loads are issued before
+// this one's arithmetic (25 float and 25 double multiply-adds an output).
+// 300 x 300 x 1369, 25 taps: 555 us; 630 without the loads ahead, 620 in two passes.
+__global__ void __launch_bounds__(kDotThreads) conv_bwd_rows_kernel(
+    const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out, int n_axis,
+    const float* __restrict__ rev, const double* __restrict__ dtaps, int n_taps, int start,
+    int64_t n_seg, int seg, int64_t n_items, double* __restrict__ partial) {
+  __shared__ __align__(16) float la[kSeg + kHalo + 8];
+  __shared__ __align__(16) float lb[kSeg + kHalo + 8];
+  __shared__ __align__(16) float tap[kHalo + 1];
+  __shared__ __align__(16) double dtap[kHalo + 1];
+  __shared__ double sm[kDotThreads];
+  double acc = 0.0;
+  stage_taps(tap, rev, n_taps);
+  stage_taps(dtap, dtaps, n_taps);
+  const int rstart = n_taps - 1 - start;
+  // the next item's segments are loaded while this one's are worked on
+  float na[kRowLoads], nb[kRowLoads];
+  auto geometry = [&](int64_t item, int64_t* o, int* x0, int* len) {
+    *o = item / n_seg;
+    *x0 = int(item - *o * n_seg) * seg;
+    *len = n_axis - *x0 < seg ? n_axis - *x0 : seg;
+    return (*len + 3) / 4 * 4 + n_taps - 1;
+  };
+  int64_t o;
+  int x0, len;
+  if (blockIdx.x < n_items) {
+    const int span = geometry(blockIdx.x, &o, &x0, &len);
+    load_row(na, a + o * n_axis, x0 + rstart - (n_taps - 1), span, n_axis);
+    load_row(nb, b + o * n_axis, x0 + start - (n_taps - 1), span, n_axis);
+  }
+  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const int span = geometry(item, &o, &x0, &len);
+    __syncthreads();
+    store_row(la, na, span);
+    store_row(lb, nb, span);
+    __syncthreads();
+    if (item + gridDim.x < n_items) {
+      int64_t on;
+      int xn, ln;
+      const int sn = geometry(item + gridDim.x, &on, &xn, &ln);
+      load_row(na, a + on * n_axis, xn + rstart - (n_taps - 1), sn, n_axis);
+      load_row(nb, b + on * n_axis, xn + start - (n_taps - 1), sn, n_axis);
+    }
+    const int v = 4 * threadIdx.x;
+    if (v >= len) continue;
+    float r[4];
+    row_conv4<float>(la, v, tap, n_taps, r);
+    double c[4];
+    row_conv4<double>(lb, v, dtap, n_taps, c);
+    float* dst = out + o * n_axis + x0 + v;
+    const float* av = la + v + start;  // a[x0 + v]: la starts at x0 - start
+    if (v + 4 <= len) {
+      *reinterpret_cast<Float4u*>(dst) = {{r[0], r[1], r[2], r[3]}};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc += double(av[e]) * c[e];
+    } else {
+      for (int e = 0; v + e < len; ++e) {
+        dst[e] = e == 0 ? r[0] : (e == 1 ? r[1] : r[2]);
+        acc += double(av[e]) * (e == 0 ? c[0] : (e == 1 ? c[1] : c[2]));
+      }
+    }
+  }
+  block_partial(acc, sm, partial);
+}
+
 // sum(a * conv(b)) per block over tiled items (as conv_tile_kernel), double
 // taps.  Each thread adds its outputs' a * conv(b) in item order.
 __global__ void __launch_bounds__(kDotThreads) conv_dot_tile_kernel(
@@ -494,8 +660,11 @@ __global__ void __launch_bounds__(kDotThreads) conv_dot_partial_kernel(
   if (threadIdx.x == 0) partial[blockIdx.x] = sm[0];
 }
 
+// result = the sum of the block partials in a fixed order, plus `add` (nullable);
+// result32 (nullable) = the same in float.
 __global__ void __launch_bounds__(kDotThreads) dot_final_kernel(const double* __restrict__ partial,
-                                                                int nblk, double* __restrict__ result) {
+                                                                int nblk, const double* add,
+                                                                double* result, float* result32) {
   __shared__ double sm[kDotThreads];
   double acc = 0.0;
   for (int k = threadIdx.x; k < nblk; k += kDotThreads) acc += partial[k];
@@ -505,7 +674,11 @@ __global__ void __launch_bounds__(kDotThreads) dot_final_kernel(const double* __
     if (threadIdx.x < off) sm[threadIdx.x] += sm[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *result = sm[0];
+  if (threadIdx.x == 0) {
+    const double r = add ? *add + sm[0] : sm[0];
+    *result = r;
+    if (result32) *result32 = float(r);
+  }
 }
 
 // ------------------------------------------------------------ Gaussian taps
@@ -875,6 +1048,44 @@ __global__ void __launch_bounds__(kDotThreads) conv_batch_dot_cols_kernel(
   block_partial(acc, sm, partial);
 }
 
+// conv_batch_cols_kernel and conv_batch_dot_cols_kernel of the adjoint in one
+// pass over a and b.
+template <int M>
+__global__ void __launch_bounds__(kDotThreads) conv_batch_bwd_cols_kernel(
+    const float* __restrict__ a, const float* __restrict__ bsrc, float* __restrict__ out,
+    const rbx_galaxy* __restrict__ gal, int n_gal, int n_rows, int nt, int axis,
+    const float* __restrict__ rev, const double* __restrict__ dtaps, double* __restrict__ partial) {
+  __shared__ int lines[kBatchGalMax + 1];
+  __shared__ int part[256];
+  __shared__ double sm[kDotThreads];
+  const bool packed = batch_line_prefix(gal, n_gal, n_rows, lines, part);
+  double acc = 0.0;
+  constexpr int start = (M - 1) / 2;
+  if (!packed) {
+    const int n_chunks = (nt + kLineChunk - 1) / kLineChunk;
+    const int64_t n_items = int64_t(n_rows) * n_chunks;
+    for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x)
+      batch_row_item(a, out, gal, n_gal, n_rows, nt, axis, rev, M, start, n_chunks, item);
+    acc = batch_row_dots(a, bsrc, gal, n_gal, n_rows, nt, axis, dtaps, M, start);
+  } else {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_lblk = (nt + 63) / 64;
+    const int64_t n_items = int64_t(lines[n_gal]) * n_lblk;
+    for (int64_t item = int64_t(blockIdx.x) * 4 + w; item < n_items; item += int64_t(gridDim.x) * 4) {
+      const int L = int(item / n_lblk);
+      const int l = int(item - int64_t(L) * n_lblk) * 64 + lane;
+      const bool ok = l < nt;
+      const BatchLine b = uniform_line(batch_line(gal, lines, n_gal, nt, axis, L));
+      const int64_t e0 = b.base + (ok ? l : 0);
+      acc += column_walk_bwd<M>(a + e0, bsrc + e0, b.stride, b.nb, ok, 0, b.nb, rev, dtaps,
+                                [&](int u, float v) {
+                                  if (ok) out[e0 + u * b.stride] = v;
+                                });
+    }
+  }
+  block_partial(acc, sm, partial);
+}
+
 // sum(a * conv(b)) per block: line items of a packed table as
 // conv_batch_tile_kernel, else the row items of conv_batch_dot_partial_kernel.
 __global__ void __launch_bounds__(kDotThreads) conv_batch_dot_tile_kernel(
@@ -1053,7 +1264,8 @@ int conv_axis(const float* in, float* out, int64_t n_outer, int n_axis, int64_t 
 static int conv_axis_dot(const float* a, const float* b, int64_t n_outer, int n_axis,
                          int64_t n_inner, const double* taps, int n_taps, int start,
                          double* partial, int nblk, double* result, hipStream_t s,
-                         const char* who) {
+                         const char* who, const double* add = nullptr,
+                         float* result32 = nullptr) {
   if (n_inner == 1 && n_taps - 1 <= kHalo) {
     const int seg = row_seg(n_axis);
     const int64_t n_seg = (n_axis + seg - 1) / seg;
@@ -1079,7 +1291,41 @@ static int conv_axis_dot(const float* a, const float* b, int64_t n_outer, int n_
     hipLaunchKernelGGL(conv_dot_partial_kernel, dim3(nblk), dim3(kDotThreads), 0, s, a, b, n_outer,
                        n_axis, n_inner, taps, n_taps, start, partial);
   }
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk, result);
+  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk, add, result,
+                     result32);
+  return check_launch(who);
+}
+
+// Adjoint of conv_axis (taps whose reversal is `rev`, from `start`) and its
+// sigma dot: out = conv(a, rev) from m - 1 - start, result = add + sum(a *
+// conv(b, dtaps)).  One pass over a and b for the LSF and for centred kernels
+// of the instantiated sizes, else the two passes.
+static int conv_axis_bwd(const float* a, const float* b, float* out, int64_t n_outer, int n_axis,
+                         int64_t n_inner, const float* rev, const double* dtaps, int m, int start,
+                         double* partial, int nblk, const double* add, double* result,
+                         float* result32, hipStream_t s, const char* who) {
+  if (n_inner == 1 && m - 1 <= kHalo && start >= 0 && start < m) {
+    const int seg = row_seg(n_axis);
+    const int64_t n_seg = (n_axis + seg - 1) / seg;
+    hipLaunchKernelGGL(conv_bwd_rows_kernel, dim3(nblk), dim3(kDotThreads), 0, s, a, b, out, n_axis,
+                       rev, dtaps, m, start, n_seg, seg, n_outer * n_seg, partial);
+  } else if (n_inner > 1 && 2 * start == m - 1 && m <= 15 && with_taps(m, [&](auto mc) {
+               constexpr int M = decltype(mc)::value;
+               if constexpr (M <= 15) {
+                 const ColItems c = col_items(n_outer, n_axis, n_inner);
+                 hipLaunchKernelGGL(conv_bwd_cols_kernel<M>, dim3(nblk), dim3(kDotThreads), 0, s, a,
+                                    b, out, n_axis, n_inner, rev, dtaps, c.n_blocks, c.n_segs, c.seg,
+                                    c.n_items, partial);
+               }
+             })) {
+  } else {
+    int rc = conv_axis(a, out, n_outer, n_axis, n_inner, rev, m, m - 1 - start, s);
+    if (!rc) rc = conv_axis_dot(a, b, n_outer, n_axis, n_inner, dtaps, m, start, partial, nblk, result,
+                                s, who, add, result32);
+    return rc;
+  }
+  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk, add, result,
+                     result32);
   return check_launch(who);
 }
 
@@ -1108,6 +1354,29 @@ static int scratch_ptr(double** out, const char* who) {
   }
   *out = static_cast<double*>(ptrs[dev]);
   return RBX_OK;
+}
+
+// Block partials of sum(a * conv_batch(b)).
+static int batch_dot_partials(const float* a, const float* b, const rbx_galaxy* galaxies, int32_t n_gal,
+                              int32_t n_rows, int32_t n_target, int32_t axis, const double* taps,
+                              int32_t n_taps, int32_t start, double* partial, int nblk,
+                              hipStream_t s) {
+  if (n_gal <= kBatchGalMax && with_taps(n_taps, [&](auto m) {
+        hipLaunchKernelGGL(conv_batch_dot_cols_kernel<decltype(m)::value>, dim3(nblk),
+                           dim3(kDotThreads), 0, s, a, b, galaxies, n_gal, n_rows, n_target, axis,
+                           taps, start, partial);
+      })) {
+  } else if (n_gal <= kBatchGalMax) {
+    hipLaunchKernelGGL(conv_batch_dot_tile_kernel, dim3(nblk), dim3(kDotThreads),
+                       size_t(kBatchTileAxis) * 64 * sizeof(float), s, a, b, galaxies, n_gal,
+                       n_rows, n_target, axis, taps, n_taps, start, partial);
+  } else {
+    const int n_chunks = (n_target + kLineChunk - 1) / kLineChunk;
+    hipLaunchKernelGGL(conv_batch_dot_partial_kernel, dim3(nblk), dim3(kDotThreads), 0, s, a, b,
+                       galaxies, n_gal, n_rows, n_target, axis, taps, n_taps, start, n_chunks,
+                       int64_t(n_rows) * n_chunks, partial);
+  }
+  return check_launch("rbx_conv_batch_dot");
 }
 
 }  // namespace rbx
@@ -1203,6 +1472,24 @@ int rbx_conv_axis_dot_noalloc(const float* a, const float* b, int64_t n_outer, i
                        as_stream(stream), who);
 }
 
+int rbx_conv_axis_bwd(const float* dout, const float* in, float* din, int64_t n_outer,
+                      int32_t n_axis, int64_t n_inner, const float* reversed, const double* dtaps,
+                      int32_t n_taps, int32_t start, const double* add, double* result,
+                      float* result32, void* workspace, size_t workspace_bytes, void* stream) {
+  using namespace rbx;
+  if (!dout || !in || !din || !reversed || !dtaps || !result || n_outer < 0 || n_axis < 1 ||
+      n_inner < 1 || n_taps < 1)
+    return fail(RBX_EINVAL, "rbx_conv_axis_bwd: bad arguments");
+  if (din == dout || din == in)
+    return fail(RBX_EINVAL, "rbx_conv_axis_bwd: in-place convolution not supported");
+  const int nblk = dot_blocks(n_outer * n_axis * n_inner);
+  if (!workspace || workspace_bytes < size_t(nblk) * sizeof(double))
+    return fail(RBX_EWORKSPACE, "rbx_conv_axis_bwd: workspace too small");
+  return conv_axis_bwd(dout, in, din, n_outer, n_axis, n_inner, reversed, dtaps, n_taps, start,
+                       static_cast<double*>(workspace), nblk, add, result, result32,
+                       as_stream(stream), "rbx_conv_axis_bwd");
+}
+
 int rbx_conv_batch(const float* in, float* out, const rbx_galaxy* galaxies, int32_t n_gal,
                    int32_t n_rows, int32_t n_target, int32_t axis, const float* taps,
                    int32_t n_taps, int32_t start, void* stream) {
@@ -1248,23 +1535,49 @@ int rbx_conv_batch_dot(const float* a, const float* b, const rbx_galaxy* galaxie
     return fail(RBX_EWORKSPACE, "rbx_conv_batch_dot: workspace too small");
   hipStream_t s = as_stream(stream);
   double* partial = static_cast<double*>(workspace);
-  if (n_gal <= kBatchGalMax && with_taps(n_taps, [&](auto m) {
-        hipLaunchKernelGGL(conv_batch_dot_cols_kernel<decltype(m)::value>, dim3(nblk),
-                           dim3(kDotThreads), 0, s, a, b, galaxies, n_gal, n_rows, n_target, axis,
-                           taps, start, partial);
-      })) {
-  } else if (n_gal <= kBatchGalMax) {
-    hipLaunchKernelGGL(conv_batch_dot_tile_kernel, dim3(nblk), dim3(kDotThreads),
-                       size_t(kBatchTileAxis) * 64 * sizeof(float), s, a, b, galaxies, n_gal,
-                       n_rows, n_target, axis, taps, n_taps, start, partial);
-  } else {
-    const int n_chunks = (n_target + kLineChunk - 1) / kLineChunk;
-    hipLaunchKernelGGL(conv_batch_dot_partial_kernel, dim3(nblk), dim3(kDotThreads), 0, s, a, b,
-                       galaxies, n_gal, n_rows, n_target, axis, taps, n_taps, start, n_chunks,
-                       int64_t(n_rows) * n_chunks, partial);
-  }
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk, out);
+  if (int rc = batch_dot_partials(a, b, galaxies, n_gal, n_rows, n_target, axis, taps, n_taps, start,
+                                  partial, nblk, s))
+    return rc;
+  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk,
+                     nullptr, out, nullptr);
   return check_launch("rbx_conv_batch_dot");
+}
+
+int rbx_conv_batch_bwd(const float* dout, const float* in, float* din, const rbx_galaxy* galaxies,
+                       int32_t n_gal, int32_t n_rows, int32_t n_target, int32_t axis,
+                       const float* reversed, const double* dtaps, int32_t n_taps, int32_t start,
+                       const double* add, double* result, float* result32, void* workspace,
+                       size_t workspace_bytes, void* stream) {
+  using namespace rbx;
+  if (!dout || !in || !din || !galaxies || !reversed || !dtaps || !result || n_gal < 1 ||
+      n_rows < 0 || n_target < 1 || n_taps < 1 || (axis != 0 && axis != 1))
+    return fail(RBX_EINVAL, "rbx_conv_batch_bwd: bad arguments");
+  if (din == dout || din == in)
+    return fail(RBX_EINVAL, "rbx_conv_batch_bwd: in-place convolution not supported");
+  const int nblk = dot_blocks(int64_t(n_rows) * n_target);
+  if (!workspace || workspace_bytes < size_t(nblk) * sizeof(double))
+    return fail(RBX_EWORKSPACE, "rbx_conv_batch_bwd: workspace too small");
+  hipStream_t s = as_stream(stream);
+  double* partial = static_cast<double*>(workspace);
+  const bool one_pass =
+      n_gal <= kBatchGalMax && 2 * start == n_taps - 1 && n_taps <= 15 && with_taps(n_taps, [&](auto mc) {
+        constexpr int M = decltype(mc)::value;
+        if constexpr (M <= 15)
+          hipLaunchKernelGGL(conv_batch_bwd_cols_kernel<M>, dim3(nblk), dim3(kDotThreads), 0, s, dout,
+                             in, din, galaxies, n_gal, n_rows, n_target, axis, reversed, dtaps,
+                             partial);
+      });
+  if (!one_pass) {
+    int rc = rbx_conv_batch(dout, din, galaxies, n_gal, n_rows, n_target, axis, reversed, n_taps,
+                            n_taps - 1 - start, stream);
+    if (rc) return rc;
+    rc = batch_dot_partials(dout, in, galaxies, n_gal, n_rows, n_target, axis, dtaps, n_taps, start,
+                            partial, nblk, s);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kDotThreads), 0, s, partial, nblk, add, result,
+                     result32);
+  return check_launch("rbx_conv_batch_bwd");
 }
 
 }  // extern "C"

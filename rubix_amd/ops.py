@@ -416,6 +416,29 @@ def conv_axis_dot(a, b, taps, n_outer, n_axis, n_inner, start):
     return res
 
 
+def conv_axis_bwd(dout, x, reversed_taps, dtaps, n_outer, n_axis, n_inner, start, add=None):
+    """Adjoint of conv_axis and its dot with the derivative taps in one pass:
+    (conv_axis(dout) with the reversed taps, add + sum(dout * conv_axis(x)) with
+    the float64 dtaps as a device float64 scalar, the same as float32)."""
+    _need_gpu(dout, x, reversed_taps, dtaps)
+    dout = _f32(dout, "dout")
+    x = _f32(x, "input")
+    reversed_taps = _f32(reversed_taps, "taps")
+    if dtaps.dtype != torch.float64:
+        raise TypeError("conv_axis_bwd dtaps must be float64")
+    dtaps = dtaps.contiguous()
+    dev = dout.device
+    din = torch.empty_like(dout)
+    wsb = max(_lib.load().rbx_dot_workspace_size(n_outer * n_axis * n_inner), 8)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    res = torch.empty((), dtype=torch.float64, device=dev)
+    res32 = torch.empty((), dtype=torch.float32, device=dev)
+    call("rbx_conv_axis_bwd", ptr(dout), ptr(x), ptr(din), n_outer, n_axis, n_inner,
+         ptr(reversed_taps), ptr(dtaps), dtaps.numel(), start, ptr(add), ptr(res), ptr(res32), ptr(ws),
+         wsb, stream_handle(dev))
+    return din, res, res32
+
+
 # ---------------------------------------------------------------- batches
 
 TUNE_TWO_PASS = 1  # rbx_tuning.flags: star_norm + per-tile accumulation forward
@@ -546,6 +569,27 @@ def conv_batch_dot(a, b, layout: BatchLayout, axis: int, taps, start: int):
          a.shape[-1], axis, ptr(taps), taps.numel(), start, ptr(res), ptr(ws), wsb,
          stream_handle(a.device))
     return res
+
+
+def conv_batch_bwd(dout, x, layout: BatchLayout, axis: int, reversed_taps, dtaps, start: int, add=None):
+    """conv_axis_bwd for one pass over every galaxy of a batch cube."""
+    _need_gpu(dout, x, reversed_taps, dtaps)
+    dout = _f32(dout, "dout")
+    x = _f32(x, "input")
+    reversed_taps = _f32(reversed_taps, "taps")
+    if dtaps.dtype != torch.float64:
+        raise TypeError("conv_batch_bwd dtaps must be float64")
+    dtaps = dtaps.contiguous()
+    dev = dout.device
+    din = torch.empty_like(dout)
+    wsb = max(_lib.load().rbx_dot_workspace_size(dout.numel()), 8)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=dev)
+    res = torch.empty((), dtype=torch.float64, device=dev)
+    res32 = torch.empty((), dtype=torch.float32, device=dev)
+    call("rbx_conv_batch_bwd", ptr(dout), ptr(x), ptr(din), ptr(layout.table), layout.n_gal,
+         layout.n_rows, dout.shape[-1], axis, ptr(reversed_taps), ptr(dtaps), dtaps.numel(), start,
+         ptr(add), ptr(res), ptr(res32), ptr(ws), wsb, stream_handle(dev))
+    return din, res, res32
 
 
 # ---------------------------------------------------------------- per step
