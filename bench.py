@@ -180,7 +180,7 @@ LAUNCH_KERNELS = {
             "star_prep_kernel", "chunk_count_kernel", "chunk_fill_kernel", "cube_fused_kernel",
             "star_norm_kernel", "star_sf_kernel", "cube_accum_kernel", "cube_combine_kernel"),
     "bwd": ("star_bwd_reg_kernel", "star_bwd_kernel", "star_grad_kernel"),
-    "noise_fwd": ("flux_rows_kernel", "noise_s2n_kernel", "add_noise_kernel"),
+    "noise_fwd": ("flux_rows_kernel", "noise_median_kernel", "add_noise_kernel"),
     "noise_bwd": ("noise_bwd_rows_kernel", "noise_coef_kernel", "add_rows_kernel"),
 }
 
