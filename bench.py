@@ -179,7 +179,7 @@ LAUNCH_KERNELS = {
             "sort_scatter_kernel", "scan_reduce_kernel", "scan_top_kernel", "scan_down_kernel", "sort_offsets_kernel",
             "star_prep_kernel", "chunk_count_kernel", "chunk_fill_kernel", "cube_fused_kernel",
             "star_norm_kernel", "star_sf_kernel", "cube_accum_kernel", "cube_combine_kernel"),
-    "bwd": ("star_bwd_reg_kernel", "star_bwd_kernel", "star_grad_kernel"),
+    "bwd": ("star_bwd_reg_kernel", "star_bwd_run_kernel", "star_bwd_kernel", "star_grad_kernel"),
     "noise_fwd": ("flux_rows_kernel", "noise_median_kernel", "add_noise_kernel"),
     "noise_bwd": ("noise_bwd_rows_kernel", "noise_coef_kernel", "add_rows_kernel"),
 }
@@ -243,6 +243,9 @@ def summarize_counters(args):
                     ks[k]["valu2_per_wave"] = e["SQ_ACTIVE_INST_VALU2"] / e["SQ_WAVES"]
                 if "SQ_INSTS_VALU_INT32" in e:
                     ks[k]["int32_per_wave"] = e["SQ_INSTS_VALU_INT32"] / e["SQ_WAVES"]
+        # a noise launch has one instantiation of each kernel
+        if kind.startswith("noise"):
+            ks = {k.split("<")[0]: e for k, e in ks.items()}
         launches[name] = {"kernels": ks}
     label = args.workload_label or args.workload
     data = {"workload": label, "launches": launches,
