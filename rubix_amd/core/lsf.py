@@ -8,6 +8,7 @@ import torch
 
 from ..autograd import GaussianLSF, lsf_x
 from ..logger import get_logger
+from ..ops import device_number
 from .data import RubixData
 from .telescope import get_telescope
 
@@ -32,7 +33,7 @@ def get_convolve_lsf(config: dict) -> Callable:
         """Convolve the input datacube with the LSF."""
         logger.info("Convolving with LSF...")
         cube = rubixdata.stars.datacube
-        s = sigma if torch.is_tensor(sigma) else torch.tensor(float(sigma), device=cube.device)
+        s = sigma if torch.is_tensor(sigma) else device_number(sigma, (), cube.device)
         rubixdata.stars.datacube = GaussianLSF.apply(cube, s, wave_resolution)
         return rubixdata
 

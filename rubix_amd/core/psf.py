@@ -8,6 +8,7 @@ import torch
 
 from ..autograd import GaussianPSF
 from ..logger import get_logger
+from ..ops import device_number
 from .data import RubixData
 
 
@@ -31,7 +32,7 @@ def get_convolve_psf(config: dict) -> Callable:
         """Convolve the input datacube with the PSF kernel."""
         logger.info("Convolving with PSF...")
         cube = rubixdata.stars.datacube
-        s = sigma if torch.is_tensor(sigma) else torch.tensor(float(sigma), device=cube.device)
+        s = sigma if torch.is_tensor(sigma) else device_number(sigma, (), cube.device)
         rubixdata.stars.datacube = GaussianPSF.apply(cube, s, size)
         return rubixdata
 

@@ -36,6 +36,19 @@ def _f32(t, name):
     return t.contiguous()
 
 
+_F32_MAX = torch.finfo(torch.float32).max
+
+
+def device_number(value, shape, device, dtype=None):
+    """A tensor of `shape` filled with a python number, as torch.tensor rounds it,
+    written by a kernel: a copy from pageable memory makes the host wait (18 us,
+    a fill 6) and cannot be captured into a graph."""
+    value = float(value)
+    if abs(value) <= _F32_MAX:
+        return torch.full(shape, value, dtype=dtype, device=device)
+    return torch.tensor(value, dtype=dtype, device=device).expand(shape).contiguous()  # inf, nan
+
+
 # ---------------------------------------------------------------- spaxels
 
 def spaxel_assign(coords: torch.Tensor, edges: torch.Tensor) -> torch.Tensor:
@@ -363,11 +376,11 @@ def gauss_taps(x, sigma):
         sigma = sigma.to(torch.float64)
     x = x.contiguous()
     n = x.numel()
-    taps = torch.empty(2, n, dtype=torch.float32, device=x.device)
+    taps, rev = torch.empty(2, n, dtype=torch.float32, device=x.device).unbind(0)
     dtaps = torch.empty(n, dtype=torch.float64, device=x.device)
-    call("rbx_gauss_taps", ptr(x), n, ptr(sigma), int(sigma.dtype == torch.float64), ptr(taps[0]),
-         ptr(taps[1]), ptr(dtaps), stream_handle(x.device))
-    return taps[0], taps[1], dtaps
+    call("rbx_gauss_taps", ptr(x), n, ptr(sigma), int(sigma.dtype == torch.float64), ptr(taps),
+         ptr(rev), ptr(dtaps), stream_handle(x.device))
+    return taps, rev, dtaps
 
 
 def conv_axis(x, taps, n_outer, n_axis, n_inner, start):
@@ -786,8 +799,11 @@ def apply_noise(cube, signal_to_noise, distribution: str = "normal", seed: int =
     _need_gpu(cube)
     code = _noise_code(distribution)
     cube, n_spaxel, nt = _cube_rows(cube)
-    sn = torch.as_tensor(signal_to_noise, dtype=torch.float32, device=cube.device)
-    sn = torch.broadcast_to(sn, cube.shape[:-1]).contiguous()
+    if isinstance(signal_to_noise, (int, float)):
+        sn = device_number(signal_to_noise, cube.shape[:-1], cube.device, torch.float32)
+    else:
+        sn = torch.as_tensor(signal_to_noise, dtype=torch.float32, device=cube.device)
+        sn = torch.broadcast_to(sn, cube.shape[:-1]).contiguous()
     dev = cube.device
     flux = torch.empty(cube.shape[:-1], dtype=torch.float32, device=dev)
     s2n = torch.empty_like(flux)
