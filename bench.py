@@ -176,8 +176,8 @@ def roofline_of(counters, call, call_ms, algo_bytes):
 # Kernels of each C-ABI launch (name prefixes after the namespace).
 LAUNCH_KERNELS = {
     "fwd": ("band_key_kernel", "batch_keys_kernel", "fill_i32_kernel", "sort_rank_kernel", "sort_tile_kernel",
-            "sort_scatter_kernel", "scan_reduce_kernel", "scan_top_kernel", "scan_down_kernel", "sort_offsets_kernel",
-            "star_prep_kernel", "chunk_count_kernel", "chunk_fill_kernel", "cube_fused_kernel",
+            "sort_scatter_kernel", "scan_reduce_kernel", "scan_top_kernel", "scan_down_kernel",
+            "star_prep_kernel", "chunk_plan_kernel", "chunk_count_kernel", "chunk_fill_kernel", "cube_fused_kernel",
             "star_norm_kernel", "star_sf_kernel", "cube_accum_kernel", "cube_combine_kernel"),
     "bwd": ("star_bwd_reg_kernel", "star_bwd_run_kernel", "star_bwd_kernel", "star_grad_kernel"),
     "noise_fwd": ("flux_rows_kernel", "noise_median_kernel", "add_noise_kernel"),

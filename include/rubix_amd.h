@@ -48,6 +48,10 @@ int rbx_spaxel_assign(const float* coords, int64_t n, int64_t stride,
                       const float* edges, int32_t n_edges, int32_t* out_ids,
                       void* stream);
 
+/* out (n, cols) row-major: v in column `col`, zeros elsewhere. */
+int rbx_column_rows(const float* v, int64_t n, int32_t cols, int32_t col,
+                    float* out, void* stream);
+
 /* Stable sort-by-spaxel index (new; the reference analogue is the lexsort +
  * searchsorted at rubix/spectra/dust/dust_extinction.py:237-267).
  *   perm     (n)          stable argsort of ids (ids outside [0, n_keys) last,

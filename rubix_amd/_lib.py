@@ -68,6 +68,7 @@ SIGNATURES = {
     "rbx_last_error_string": (ctypes.c_char_p, []),
     "rbx_spaxel_assign": (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int32, c_void_p, c_void_p]),
     "rbx_spaxel_sort_workspace_size": (c_size_t, [c_int64, c_int32]),
+    "rbx_column_rows": (c_int, [c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p]),
     "rbx_spaxel_sort": (c_int, [c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_size_t, c_void_p]),
     "rbx_ssp_prepare": (c_int, [POINTER(RbxSsp), c_void_p, c_void_p, c_void_p]),

@@ -118,10 +118,7 @@ class FusedDatacube(torch.autograd.Function):
         need = ctx.needs_input_grad
         dm, dt, dz, dv = ops.cube_backward(ctx.ssp, ctx.target, ctx.cctx, dcube.contiguous(),
                                            need=(need[0], need[1], need[2], need[3]))
-        dvel = None
-        if need[3]:
-            dvel = torch.zeros(ctx.vshape, dtype=torch.float32, device=dcube.device)
-            dvel.select(1, ctx.vel_comp).copy_(dv)
+        dvel = ops.column_rows(dv, ctx.vshape, ctx.vel_comp) if need[3] else None
         return dm, dt, dz, dvel, None, None, None, None, None, None, None, None
 
 
@@ -303,10 +300,7 @@ class BatchedDatacube(torch.autograd.Function):
         need = ctx.needs_input_grad
         dm, dt, dz, dv = ops.batch_backward(ssp, target, layout, ctx.cctx, dcube.contiguous(),
                                             need=(need[0], need[1], need[2], need[3]), tune=tune)
-        dvel = None
-        if need[3]:
-            dvel = torch.zeros(ctx.vshape, dtype=torch.float32, device=dcube.device)
-            dvel.select(1, vel_comp).copy_(dv)
+        dvel = ops.column_rows(dv, ctx.vshape, vel_comp) if need[3] else None
         return dm, dt, dz, dvel, None, None, None, None, None, None, None
 
 
@@ -408,10 +402,7 @@ class Resample(torch.autograd.Function):
         need_s, need_v = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         ds, dv = ops.resample_bwd(ssp, target, spectra, vel, dout.contiguous(), vel_comp, c,
                                   need_spectra=need_s, need_velocity=need_v)
-        dvel = None
-        if need_v:
-            dvel = torch.zeros_like(vel)
-            dvel.select(1, vel_comp).copy_(dv)
+        dvel = ops.column_rows(dv, vel.shape, vel_comp) if need_v else None
         return ds, dvel, None, None, None, None
 
 

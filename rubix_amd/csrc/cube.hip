@@ -526,6 +526,46 @@ __global__ void chunk_count_kernel(const int32_t* __restrict__ offsets, int32_t 
   }
 }
 
+// chunk_count_kernel, the scan and chunk_fill_kernel for up to kPlanKeys keys:
+// one workgroup, a stretch of keys a thread.  Each of the three is a launch
+// of some 2 us of work.
+constexpr int kPlanThreads = 1024;
+constexpr int kPlanKeys = 8 * kPlanThreads;
+
+__global__ void __launch_bounds__(kPlanThreads) chunk_plan_kernel(
+    const int32_t* __restrict__ offsets, int32_t ns, int chunk, int32_t* __restrict__ chunk_off,
+    ChunkDesc* __restrict__ desc) {
+  __shared__ int32_t wave_sum_s[kPlanThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int per = (ns + kPlanThreads - 1) / kPlanThreads;
+  const int p0 = tid * per < ns ? tid * per : ns, p1 = p0 + per < ns ? p0 + per : ns;
+  int32_t own = 0;
+  for (int p = p0; p < p1; ++p) own += (offsets[p + 1] - offsets[p] + chunk - 1) / chunk;
+  int32_t incl = own;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t t = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += t;
+  }
+  if (lane == 63) wave_sum_s[w] = incl;
+  __syncthreads();
+  int32_t o = incl - own;
+  for (int v = 0; v < w; ++v) o += wave_sum_s[v];
+  if (tid == kPlanThreads - 1) chunk_off[ns] = o + own;
+  for (int p = p0; p < p1; ++p) {
+    chunk_off[p] = o;
+    const int32_t b = offsets[p], e = offsets[p + 1];
+    for (int32_t s = b; s < e; s += chunk, ++o) {
+      ChunkDesc d;
+      d.spaxel = int32_t(p);
+      d.begin = s;
+      d.end = s + chunk < e ? s + chunk : e;
+      d.pad = 0;
+      desc[o] = d;
+    }
+  }
+}
+
 __global__ void chunk_fill_kernel(const int32_t* __restrict__ offsets, int32_t n_spaxel,
                                   int chunk, const int32_t* __restrict__ chunk_off,
                                   ChunkDesc* __restrict__ desc) {
@@ -2157,6 +2197,13 @@ static int validate(const rbx_ssp* ssp, const rbx_target* tg, const rbx_stars* s
 
 int build_chunks(const int32_t* offsets, int32_t ns, int chunk, int32_t* chunk_off,
                  int32_t* scan_blocks, ChunkDesc* desc, hipStream_t s) {
+  // 10 k stars, 2500 keys: 4 us against 8 and two more launches; past kPlanKeys
+  // the one workgroup's stretches take longer than the launches
+  if (ns <= kPlanKeys) {
+    hipLaunchKernelGGL(chunk_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, offsets, ns, chunk,
+                       chunk_off, desc);
+    return check_launch("build_chunks");
+  }
   hipLaunchKernelGGL(chunk_count_kernel, dim3(grid_for(int64_t(ns) + 1, 256)), dim3(256), 0, s,
                      offsets, ns, chunk, chunk_off);
   int rc = exclusive_scan_i32(chunk_off, int64_t(ns) + 1, scan_blocks, s);

@@ -84,6 +84,17 @@ __global__ void spaxel_assign_kernel(const float* __restrict__ coords, int64_t n
   }
 }
 
+// out[i, c] = v[i] in column `col`, 0 in the others (a velocity gradient of
+// one component), one pass instead of a fill and a strided copy.
+__global__ void __launch_bounds__(256) column_rows_kernel(const float* __restrict__ v, int64_t n,
+                                                          int cols, int col,
+                                                          float* __restrict__ out) {
+  for (int64_t i = gtid(); i < n; i += int64_t(gridDim.x) * blockDim.x) {
+    const float x = v[i];
+    for (int c = 0; c < cols; ++c) out[i * cols + c] = c == col ? x : 0.f;
+  }
+}
+
 // ------------------------------------------------------------ integer scan
 
 constexpr int kScanThreads = 256;
@@ -436,12 +447,17 @@ __global__ void __launch_bounds__(1024) sort_tile_kernel(
 // pos = the star's base in the scanned table + its rank: perm[pos] = the
 // element's input index (src_perm[i], or i on the first pass), bucket_out[pos]
 // = its bucket, sorted[pos] = its original id (ids[perm[pos]]; in[i] itself on
-// the first pass).
+// the first pass), offsets[k] (where wanted) = the first position of key k, k in
+// [0, n_keys].
 __global__ void __launch_bounds__(256) sort_scatter_kernel(
     const int32_t* __restrict__ in, int64_t n, int32_t n_keys, uint32_t tile, int64_t ntiles,
     int shift, int32_t mask, const int32_t* __restrict__ table, const uint16_t* __restrict__ rank,
     const int32_t* __restrict__ src_perm, const int32_t* __restrict__ ids,
-    int32_t* __restrict__ perm, int32_t* __restrict__ bucket_out, int32_t* __restrict__ sorted) {
+    int32_t* __restrict__ perm, int32_t* __restrict__ bucket_out, int32_t* __restrict__ sorted,
+    int32_t* __restrict__ offsets) {
+  if (offsets)
+    for (int64_t k = gtid(); k <= n_keys; k += int64_t(gridDim.x) * blockDim.x)
+      offsets[k] = table[k * ntiles];
   for (int64_t i = gtid(); i < n; i += int64_t(gridDim.x) * blockDim.x) {
     const int32_t id = in[i];
     const int full = bucket_of(id, n_keys);
@@ -468,12 +484,6 @@ __global__ void bucket_offsets_kernel(const int32_t* __restrict__ ids,
     }
     offsets[k] = int32_t(lo);
   }
-}
-
-__global__ void sort_offsets_kernel(const int32_t* __restrict__ table, int32_t n_keys,
-                                    int64_t ntiles, int32_t* __restrict__ offsets) {
-  for (int64_t k = gtid(); k <= n_keys; k += int64_t(gridDim.x) * blockDim.x)
-    offsets[k] = table[k * ntiles];
 }
 
 static int grid_for(int64_t n, int threads, int64_t cap = 65536) {
@@ -551,13 +561,12 @@ static int sort_pass(const SortPlan& p, const int32_t* in, int shift, int32_t ma
   }
   int rc = exclusive_scan_i32(table, p.table, blocks, s);
   if (rc) return rc;
-  if (offsets)
-    hipLaunchKernelGGL(sort_offsets_kernel, dim3(grid_for(int64_t(p.n_keys) + 1, 256)), dim3(256),
-                       0, s, table, p.n_keys, p.ntiles, offsets);
   if (p.n > 0)
     hipLaunchKernelGGL(sort_scatter_kernel, dim3(grid_for(p.n, 256)), dim3(256), 0, s, in, p.n,
                        p.n_keys, uint32_t(p.tile), p.ntiles, shift, mask, table, rank, src_perm,
-                       ids, perm, bucket_out, sorted);
+                       ids, perm, bucket_out, sorted, offsets);
+  else if (offsets)
+    fill_i32(offsets, int64_t(p.n_keys) + 1, 0, s);
   return check_launch("rbx_spaxel_sort");
 }
 
@@ -621,6 +630,16 @@ int rbx_spaxel_assign(const float* coords, int64_t n, int64_t stride, const floa
                        stride, edges, n_edges, out_ids);
   }
   return check_launch("rbx_spaxel_assign");
+}
+
+int rbx_column_rows(const float* v, int64_t n, int32_t cols, int32_t col, float* out, void* stream) {
+  using namespace rbx;
+  if (n < 0 || cols < 1 || col < 0 || col >= cols || (n > 0 && (!v || !out)))
+    return fail(RBX_EINVAL, "rbx_column_rows: bad arguments");
+  if (n == 0) return RBX_OK;
+  hipLaunchKernelGGL(column_rows_kernel, dim3(grid_for(n, 256)), dim3(256), 0,
+                     as_stream(stream), v, n, cols, col, out);
+  return check_launch("rbx_column_rows");
 }
 
 size_t rbx_spaxel_sort_workspace_size(int64_t n, int32_t n_keys) {

@@ -85,6 +85,15 @@ def spaxel_sort(ids: torch.Tensor, n_keys: int):
     return perm, srt, offsets
 
 
+def column_rows(v, shape, col: int):
+    """(n, columns) float32 with v in column col and zeros elsewhere."""
+    _need_gpu(v)
+    v = _f32(v, "column")
+    out = torch.empty(shape, dtype=torch.float32, device=v.device)
+    call("rbx_column_rows", ptr(v), shape[0], shape[1], col, ptr(out), stream_handle(v.device))
+    return out
+
+
 # ---------------------------------------------------------------- alignment
 
 def filter_particles(coords, lo: float, hi: float, *fields):
