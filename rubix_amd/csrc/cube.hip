@@ -2006,13 +2006,55 @@ struct CubeLayout {
   int64_t max_chunks;
 };
 
+// Wavefronts of a fused workgroup: 64 NB bins each.
+static int fused_waves(int nt, int nb) { return (nt + 64 * nb - 1) / (64 * nb); }
+
+// Fused workgroups the chip's 256 CUs take at once: 2 of 16 wavefronts a CU,
+// 4 of 8, 7 of 4.
+static int64_t fused_slots(int32_t nt) {
+  const int w = fused_waves(nt < 4096 ? nt : 4096, 4);
+  return 256 * (w > 8 ? 2 : (w > 4 ? 4 : 7));
+}
+
+// Stars per reduction chunk where the caller leaves it open.  A chunk's stars
+// are walked one after another (about 1 us each), so the largest chunk is the
+// tail of the launch: eight chunks for every resident workgroup keep it short,
+// at the price of one f64 partial row per chunk.  At 10 k stars -> 25 x 25 x
+// 1000 chunks of up to 256 took 183 us, one spaxel at the field's edge holding
+// most of that; now 26 us.
+static int auto_chunk(int64_t n, int32_t nt) {
+  const int64_t c = n / (8 * fused_slots(nt));
+  return c < 8 ? 8 : (c > 256 ? 256 : int(c));
+}
+
+// At least ceil(m / auto_chunk(m, nt)) for every m <= n: a chunk is n / (8
+// slots) rounded down from 9 up, so that is at most 9 slots chunks, ceil(n / 8)
+// of the shortest and ceil(n / 256) of the longest.
+static int64_t auto_chunks_room(int64_t n, int32_t nt) {
+  const int64_t most = 9 * fused_slots(nt), longest = (n + 255) / 256, shortest = (n + 7) / 8;
+  const int64_t r = longest > most ? longest : most;
+  return r < shortest ? r : shortest;
+}
+
 // per_star_only: carve just the per-star arrays (what the adjoint reads).
+// chunk 0: auto_chunk's, in a workspace that never shrinks with the star or
+// the bin count, so one sized for a program's largest call takes every other.
 template <class C>
 static void cube_layout(C& c, int64_t n, int32_t n_keys, int32_t nt, int chunk, CubeLayout* L,
                         bool per_star_only = false) {
   // sort keys band * n_spaxel + spaxel: up to band_cap(n_keys) * n_keys
   const int64_t nk = int64_t(band_cap(n_keys)) * n_keys;
-  const int64_t max_chunks = (n + chunk - 1) / chunk + nk;
+  const int len = chunk ? chunk : auto_chunk(n, nt);
+  const int64_t max_chunks = (n + len - 1) / len + nk;
+  int64_t desc_room = max_chunks, part_room = max_chunks * nt;
+  if (!chunk) {
+    // fewer bins have more slots: the room is the most of the bin counts up to nt
+    for (const int32_t b : {nt, nt < 2048 ? nt : 2048, nt < 1024 ? nt : 1024}) {
+      const int64_t rows = auto_chunks_room(n, b) + nk;
+      if (rows > desc_room) desc_room = rows;
+      if (rows * b > part_room) part_room = rows * b;
+    }
+  }
   const size_t sort_bytes = sort_workspace_bound(n, int32_t(nk));
   const size_t n1 = size_t(n > 0 ? n : 1);
   auto* perm = c.template take<int32_t>(n1);
@@ -2038,8 +2080,8 @@ static void cube_layout(C& c, int64_t n, int32_t n_keys, int32_t nt, int chunk, 
   auto* coff = c.template take<int32_t>(size_t(nk) + 1);
   auto* blocks = c.template take<int32_t>((size_t(nk) + 1) / 4096 + 2);
   auto* keys = c.template take<int32_t>(n1);
-  auto* desc = c.template take<ChunkDesc>(size_t(max_chunks > 0 ? max_chunks : 1));
-  auto* part = c.template take<double>(size_t(max_chunks > 0 ? max_chunks : 1) * nt);
+  auto* desc = c.template take<ChunkDesc>(size_t(desc_room > 0 ? desc_room : 1));
+  auto* part = c.template take<double>(size_t(part_room > 0 ? part_room : nt));
   auto* sws = c.template take<char>(sort_bytes);
   if (L) {
     L->perm = reinterpret_cast<int32_t*>(perm);
@@ -2219,9 +2261,6 @@ void combine_chunks(const double* partial, const int32_t* chunk_off, int32_t ns,
                      partial, chunk_off, ns, bands, nt, cube);
 }
 
-// Wavefronts of a fused workgroup: 64 NB bins each.
-static int fused_waves(int nt, int nb) { return (nt + 64 * nb - 1) / (64 * nb); }
-
 // Runs of bins (ascending targets) where the smallest knot spacing
 // (1 / locate_inv_h on a locator with one knot per cell) is at least 2.25 times
 // the mean bin spacing: 512 bins then span at most 237 knots with the
@@ -2231,23 +2270,10 @@ static bool sparse_knots(const rbx_ssp& ssp, const rbx_target& tg) {
          float(tg.n - 1) >= 2.25f * ssp.locate_inv_h * (tg.wmax - tg.wmin);
 }
 
-// Stars per reduction chunk where the caller leaves it open.  A chunk's stars
-// are walked one after another (about 1 us each), so the largest chunk is the
-// tail of the launch: eight chunks for every resident workgroup (2 of 16
-// wavefronts a CU, 4 of 8, 7 of 4) keep it short, at the price of one f64
-// partial row per chunk.  At 10 k stars -> 25 x 25 x 1000 chunks of up to 256
-// took 183 us, one spaxel at the field's edge holding most of that; now 26 us.
-static int auto_chunk(int64_t n, int32_t nt) {
-  const int w = fused_waves(nt < 4096 ? nt : 4096, 4);
-  const int64_t slots = 256 * (w > 8 ? 2 : (w > 4 ? 4 : 7));  // of the chip's 256 CUs
-  const int64_t c = n / (8 * slots);
-  return c < 8 ? 8 : (c > 256 ? 256 : int(c));
-}
-
 size_t cube_workspace_impl(int64_t n, int32_t n_keys, int32_t nt, const Tune& t) {
   if (n < 0 || n_keys < 1 || nt < 1) return 0;
   SizeOnly so;
-  cube_layout(so, n, n_keys, nt, t.chunk ? t.chunk : auto_chunk(n, nt), nullptr);
+  cube_layout(so, n, n_keys, nt, t.chunk, nullptr);
   return so.s.used;
 }
 
@@ -2293,7 +2319,7 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   Carver c(workspace, workspace_bytes);
   CubeLayout L;
   const int chunk = t.chunk ? t.chunk : auto_chunk(n, nt);
-  cube_layout(c, n, stars->n_keys, nt, chunk, &L);
+  cube_layout(c, n, stars->n_keys, nt, t.chunk, &L);
   if (!c.ok) return failf(RBX_EWORKSPACE, "%s: workspace too small", who);
   const SspView g = view_of(*ssp);
   const int32_t ns = stars->n_spaxel;

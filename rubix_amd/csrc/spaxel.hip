@@ -218,7 +218,7 @@ struct SortPlan {
   int64_t tile;     // stars per tile, multiple of 64
   int64_t ntiles;
   int64_t table;    // (buckets or digit buckets) * ntiles
-  int64_t nblk;     // scan blocks over the table
+  int64_t room;     // table entries of the workspace: no fewer for more stars
   int nbits;        // bits needed to tell buckets apart
   int digit_bits;   // 0: one pass over all buckets; else radix digits of this width
   int passes;       // counting-sort passes
@@ -264,6 +264,26 @@ static bool plan_workgroup(SortPlan* p, int64_t buckets) {
   return true;
 }
 
+// Table entries the workspace has for `buckets` keys in one pass.  The tiles
+// grow with the star count, so the table of more stars can be the smaller one;
+// this bound of both plans never shrinks, and a workspace sized for the most
+// stars of a program takes every smaller call.
+static int64_t table_room(int64_t n, int64_t buckets) {
+  int64_t w = kTileLds / (4 * ((buckets + 1) / 2));
+  int64_t tiles;
+  if (w >= 2) {  // plan_workgroup: at most 512 tiles until its largest ones
+    if (w > 16) w = 16;
+    if (w > 4) w &= ~int64_t(3);
+    const int64_t least = (n + 64 * w - 1) / (64 * w), most = (n + 1024 * w - 1) / (1024 * w);
+    tiles = most > 512 ? most : (least < 512 ? least : 512);
+  } else {  // plan_tile: n / tile before its rounding, which adds less than one
+    const double t = sqrt(2.56e-4 * double(buckets) * double(n));
+    tiles = int64_t(double(n) / (t > double(kSortTile) ? double(kSortTile) : (t < 64 ? 64. : t))) + 2;
+  }
+  if (tiles < 1) tiles = 1;
+  return buckets * tiles < kTableCap ? buckets * tiles : kTableCap;
+}
+
 static SortPlan make_plan(int64_t n, int32_t n_keys) {
   SortPlan p;
   p.n = n;
@@ -292,7 +312,8 @@ static SortPlan make_plan(int64_t n, int32_t n_keys) {
     p.ntiles = n > 0 ? (n + p.tile - 1) / p.tile : 1;
   }
   p.table = buckets * p.ntiles;
-  p.nblk = (p.table + kScanBlock - 1) / kScanBlock;
+  p.room = p.digit_bits ? kTableCap : table_room(n, buckets);
+  if (p.room < p.table) p.room = p.table;
   return p;
 }
 
@@ -303,8 +324,8 @@ static SortPlan make_plan(int64_t n, int32_t n_keys) {
 template <class S>
 static void sort_layout(S& c, const SortPlan& p, int32_t** table, int32_t** blocks,
                         uint16_t** rank, int32_t** tperm, int32_t** b0, int32_t** b1) {
-  auto* t = c.template take<int32_t>(p.table);
-  auto* bl = c.template take<int32_t>(p.nblk + 1);
+  auto* t = c.template take<int32_t>(p.room);
+  auto* bl = c.template take<int32_t>((p.room + kScanBlock - 1) / kScanBlock + 1);
   const int64_t n1 = p.n > 0 ? p.n : 1;
   const int64_t rn = p.digit_bits ? n1 : 0;
   auto* tp = c.template take<int32_t>(rn);
@@ -526,8 +547,7 @@ size_t sort_workspace_size(int64_t n, int32_t n_keys) {
 // would need them.
 size_t sort_workspace_bound(int64_t n, int32_t max_keys) {
   SortPlan p = make_plan(n, max_keys);
-  p.table = kTableCap;
-  p.nblk = (p.table + kScanBlock - 1) / kScanBlock;
+  p.room = kTableCap;
   SizerAdapter a;
   sort_layout(a, p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
   return a.s.used;
