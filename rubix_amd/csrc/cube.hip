@@ -642,7 +642,8 @@ __global__ void __launch_bounds__(64) cube_accum_kernel(
 }
 
 // Strided bins per lane of the fused pass: NB = 4 for targets of up to 4096
-// bins (16 wavefronts x 64 lanes x 4), up to 8 for 8192.
+// bins (16 wavefronts x 64 lanes x 4; 2 or 3 where fused_bins() says), up to 8
+// for 8192.
 constexpr int kMaxFusedBins = 8;
 
 // Normalisation and accumulation in one pass for ascending targets: item q
@@ -712,9 +713,10 @@ __device__ inline float wave_sum_last(float v) {
 
 // Knots of a wavefront's staged window: 80 per bin of a lane (the 64 NB
 // bins of a wavefront span ~64 NB x 1.25 A, ~57 NB knots of a 1.4 A grid,
-// plus the margins); wider windows take the global search.
+// plus the margins); wider windows take the global search.  The layouts for
+// denser knots (fused_bins()) give the LDS of their fewer bins to the window.
 template <int NB>
-constexpr int fused_window() { return 80 * NB; }
+constexpr int fused_window() { return NB == 2 ? 448 : (NB == 3 ? 384 : 80 * NB); }
 
 // A wave-uniform float (the lanes hold the same value) in a scalar register.
 __device__ inline float uniform_f(float v) {
@@ -2270,6 +2272,25 @@ static bool sparse_knots(const rbx_ssp& ssp, const rbx_target& tg) {
          float(tg.n - 1) >= 2.25f * ssp.locate_inv_h * (tg.wmax - tg.wmin);
 }
 
+// Strided bins per lane of an axis of up to 4096 bins.  4, but where knots
+// are dense, the window of a wavefront's 256 bins does not fit its LDS (from 1.2
+// knots a bin: every bin searches memory) or takes long to stage, and 3 or 2
+// bins on more wavefronts of the same workgroup class are faster.  Forward of
+// 200 k stars at 0.67, 1.0, 1.33, 1.9, 2.9 knots a bin, 4 -> 3 bins: 700 bins 333,
+// 365, 491, 510, 540 -> 331, 338, 404, 422, 519 us; 1500 bins 588, 673, 954,
+// 1027 -> 586, 607, 773, 823; 2300 bins 924, 1098, 1881 -> 905, 931, 1275; 3000
+// bins 997, 1242 -> 1063, 1119.  4 -> 2: 500 bins 301, 327, 437, 444, 452 -> 299,
+// 309, 323, 334, 402; 1900 bins 640, 754, 1168, 1189 -> 871, 934, 982, 1056.
+// Axes that need more wavefronts than the class has lose: 900 bins 357, 405,
+// 579 -> 538, 534, 617 with 3, 511, 543, 566 with 2.
+static int fused_bins(const rbx_ssp& ssp, int nt, float span) {
+  if (ssp.locate_multi || nt < 2) return 4;
+  const float knots = float(ssp.n_wave) * ssp.locate_inv_h / float(ssp.n_locate) * span / float(nt - 1);
+  if (knots >= 1.15f && knots <= 2.9f && (nt <= 512 || (nt > 1536 && nt <= 2048))) return 2;
+  if (knots >= 0.85f && (nt <= 768 || (nt > 1024 && nt <= 1536) || (nt > 2048 && nt <= 3072))) return 3;
+  return 4;
+}
+
 size_t cube_workspace_impl(int64_t n, int32_t n_keys, int32_t nt, const Tune& t) {
   if (n < 0 || n_keys < 1 || nt < 1) return 0;
   SizeOnly so;
@@ -2373,9 +2394,21 @@ int cube_fwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
       else launch_fused<8, 16, 2>(f);
     } else switch (nb_lane) {
       case 4:
-        if (w <= 4) launch_fused<4, 4>(f);
-        else if (w <= 8) launch_fused<4, 8>(f);
-        else launch_fused<4, 16>(f);
+        switch (fused_bins(*ssp, nt, target->wmax - target->wmin)) {
+          case 2:
+            if (w <= 2) launch_fused<2, 4>(f);
+            else launch_fused<2, 16>(f);
+            break;
+          case 3:
+            if (w <= 3) launch_fused<3, 4>(f);
+            else if (w <= 6) launch_fused<3, 8>(f);
+            else launch_fused<3, 16>(f);
+            break;
+          default:
+            if (w <= 4) launch_fused<4, 4>(f);
+            else if (w <= 8) launch_fused<4, 8>(f);
+            else launch_fused<4, 16>(f);
+        }
         break;
       case 5: launch_fused<5, 16>(f); break;
       case 6: launch_fused<6, 16>(f); break;
