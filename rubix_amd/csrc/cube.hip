@@ -1865,6 +1865,149 @@ __global__ void __launch_bounds__(64 * W) star_bwd_run_kernel(
   }
 }
 
+// star_bwd_run_kernel's records for knots denser than bins (dense_knots()),
+// where 64 bins span more than the 64 knots that star_bwd_reg_kernel holds one per
+// lane: groups of 64 bins, one per lane, each searching its exact segment among the
+// group's records.  The next group's bins are loaded before this one's
+// records are staged.  Adjoint call of 200 k stars at 1.0, 1.33, 1.9 knots a
+// bin, with bins gathered from memory before: 500 bins 453, 497, 500 -> 345, 360,
+// 451 us; 1500 bins 1180, 1333, 1338 -> 874, 899, 1153; 2300 bins at 1.0 and
+// 1.33 1725, 1971 -> 1273, 1370.  Groups at a grid end, wider than the record
+// space, or with a bin outside it are gathered.
+constexpr int kBwdDenseKnots = 190;  // three rounds of 63 and the last
+
+template <int W, bool kDust>
+__global__ void __launch_bounds__(64 * W) star_bwd_dense_kernel(
+    SspView g, rbx_target tg, int64_t n, int64_t n_items, const StarState* __restrict__ state,
+    const float* __restrict__ gradw, const float* __restrict__ dcube, int slab_bins,
+    const float* __restrict__ axav, float* __restrict__ vpart, double* __restrict__ apart) {
+  constexpr int kN = kBwdDenseKnots;
+  constexpr int kBuf = kRunFields * kN + 2;  // a multiple of 16 bytes
+  static_assert(kBuf >= kRedFloats, "the lane sums reuse the record space");
+  __shared__ __align__(16) float buf_s[W][kBuf];
+  for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+    const SlabTask t = slab_task<W, kBwdSlabs>(item);
+    const bool live = t.r < n;
+    float* buf = buf_s[t.wave];
+    float v[7];
+#pragma unroll
+    for (int q = 0; q < 7; ++q) v[q] = 0.f;
+    StarState s;
+    s.row = -1;
+    if (live) s = state[t.r];
+    const uint32_t j0 = uint32_t(t.slab * slab_bins);
+    const uint32_t j1 = j0 + slab_bins < uint32_t(tg.n) ? j0 + slab_bins : uint32_t(tg.n);
+    if (s.row >= 0 && j0 < j1) {
+      const Rows R = rows_of(g, __builtin_amdgcn_readfirstlane(s.row));
+      const float* grow = dcube + int64_t(__builtin_amdgcn_readfirstlane(s.spaxel)) * tg.n;
+      s.a = uniform_f(s.a);
+      s.inv_a = uniform_f(s.inv_a);
+      const Shift h = shift_of(g, s.a, s.inv_a);
+      BwdRows B;
+      B.fu = uniform_f(gradw[t.r * 2]);
+      B.fs = uniform_f(gradw[t.r * 2 + 1]);
+      float wc[4];  // the corner weights, wave-uniform
+#pragma unroll
+      for (int c = 0; c < 4; ++c) wc[c] = uniform_f(s.w[c]);
+      // a bin past the slab takes its last bin's x and weights 0
+      auto bin_of = [&](uint32_t jb) {
+        const uint32_t j = jb + uint32_t(t.lane);
+        return j < j1 ? j : j1 - 1;
+      };
+      Pair xd = ld_pair(tg.pairs, 2 * bin_of(j0));
+      float gv = ld_at(grow, bin_of(j0));
+      int k0 = loc_k0(g, xd.lo, h);
+      for (uint32_t jb = j0; jb < j1; jb += kTile) {
+        const bool in = jb + uint32_t(t.lane) < j1;
+        const float x = xd.lo, dj = in ? xd.hi : 0.f;
+        float gj = in ? gv : 0.f;
+        if (kDust && s.av != 0.f) gj *= dust_factor(dust_tau(axav, bin_of(jb)), s.av);
+        // every guess with a margin of 3 knots below and 5 above (run_values)
+        const int k_lo = __builtin_amdgcn_readfirstlane(k0) - 3;
+        const int nk = __builtin_amdgcn_readlane(k0, 63) + 5 - k_lo + 1;
+        int l = k0 - k_lo;  // in [3, nk - 6]: the guesses are monotone in the bin
+        const uint32_t jn = bin_of(jb + kTile);
+        xd = ld_pair(tg.pairs, 2 * jn);
+        gv = ld_at(grow, jn);
+        bool done = false;
+        if (nk <= kN && k_lo >= 1 && k_lo + nk < g.n_wave) {
+          wave_lds_sync();  // the group before is read
+          for (int b = 0; b < nk - 1; b += 63) {
+            const int k = b + t.lane;
+            const uint32_t kk = uint32_t(k_lo + (k < nk ? k : nk - 1));
+            const float lamk = ld_at(g.wave, kk);
+            float fc[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) fc[c] = ld_at(R.f[c], kk);
+            const RowVals rv = combine_rows(fc[0], fc[1], fc[2], fc[3], B.fu, B.fs);
+            const float dwk = w_change(fc, wc);
+            const float w = mul_nocontract(lamk, s.a);
+            const float r = __builtin_amdgcn_rcpf(next_lane(w) - w);
+            const float su = (next_lane(rv.u) - rv.u) * r, ss = (next_lane(rv.s) - rv.s) * r;
+            // lane 63 repeats the next round's first knot (its slopes need
+            // the knot after it); the window's last knot is only compared
+            if (k < nk && (t.lane < 63 || k == nk - 1)) {
+              buf[kRw * kN + k] = w;
+              buf[kRRw * kN + k] = rv.w;
+              buf[kRSw * kN + k] = dwk * r;
+              buf[kRRu * kN + k] = rv.u;
+              buf[kRSu * kN + k] = su;
+              buf[kRRs * kN + k] = rv.s;
+              buf[kRSs * kN + k] = ss;
+            }
+          }
+          k0 = loc_k0(g, xd.lo, h);
+          wave_lds_sync();
+          l += buf[l + 1] <= x ? 1 : 0;
+          float wl = buf[l], wr = buf[l + 1];
+          if (__ballot(x >= wr || x < wl)) {  // rare: the exact search
+            while (x >= wr && l < nk - 2) {
+              ++l;
+              wr = buf[l + 1];
+            }
+            while (x < buf[l] && l > 0) --l;
+            wl = buf[l];
+            wr = buf[l + 1];
+          }
+          if (!__ballot(x >= wr || x < wl)) {
+            const float d = x - wl, RSw = buf[kRSw * kN + l];
+            const float Ruv = buf[kRRu * kN + l] + d * buf[kRSu * kN + l];
+            const float Rsv = buf[kRRs * kN + l] + d * buf[kRSs * kN + l];
+            v[0] += gj * (buf[kRRw * kN + l] + d * RSw);
+            v[1] += gj * Ruv;
+            v[2] += gj * Rsv;
+            v[3] += dj * Ruv;
+            v[4] += dj * Rsv;
+            const float kd = x * RSw;  // as in bwd_run
+            v[5] -= gj * kd;
+            v[6] -= dj * kd;
+            done = true;
+          }
+        } else {
+          k0 = loc_k0(g, xd.lo, h);
+        }
+        if (!done) {
+          float u[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          bwd_bin_gather(g, R, s, B, h, x, gj, dj, u);
+#pragma unroll
+          for (int e = 0; e < 5; ++e) v[e] += u[e];
+          v[5] += u[5] * s.a;
+          v[6] += u[6] * s.a;
+        }
+      }
+      v[5] *= s.inv_a;
+      v[6] *= s.inv_a;
+    }
+    const double tot = lds_sum<7>(v, buf, t.lane);
+    const int q = t.lane >> 3;
+    if (live && (t.lane & 7) == 0 && q < 7) {
+      const int64_t it = t.r * kBwdSlabs + t.slab;
+      if (q < kVSums) vpart[it * kVSums + q] = float(tot);
+      else apart[it * kASums + q - kVSums] = tot;
+    }
+  }
+}
+
 // Per star: add the slab sums in slab order and form every gradient in
 // closed form.  With P_j = m sum_c w_c R_c(j) and sf = T / Nn:
 //   sum_j g_j dP_j/dtheta = m Pg_theta, dNn/dtheta = m Pd_theta,
@@ -2190,7 +2333,16 @@ template <int W>
 static void launch_bwd(int64_t grid, hipStream_t s, const SspView& g, const rbx_target& tg,
                        int64_t n, int64_t items, const StarState* st, const float* gradw,
                        const float* dcube, int slab_bins, const float* axav, float* vp,
-                       double* ap, bool runs) {
+                       double* ap, bool runs, bool dense) {
+  if (dense) {
+    if (axav)
+      hipLaunchKernelGGL((star_bwd_dense_kernel<W, true>), dim3(grid), dim3(64 * W), 0, s, g, tg,
+                         n, items, st, gradw, dcube, slab_bins, axav, vp, ap);
+    else
+      hipLaunchKernelGGL((star_bwd_dense_kernel<W, false>), dim3(grid), dim3(64 * W), 0, s, g, tg,
+                         n, items, st, gradw, dcube, slab_bins, nullptr, vp, ap);
+    return;
+  }
   if (runs) {
     if (axav)
       hipLaunchKernelGGL((star_bwd_run_kernel<W, true>), dim3(grid), dim3(64 * W), 0, s, g, tg, n,
@@ -2272,6 +2424,22 @@ static bool sparse_knots(const rbx_ssp& ssp, const rbx_target& tg) {
          float(tg.n - 1) >= 2.25f * ssp.locate_inv_h * (tg.wmax - tg.wmin);
 }
 
+// Knots per bin on average (n_locate cells of 1 / locate_inv_h span the knots).
+static float mean_knots(const rbx_ssp& ssp, int nt, float span) {
+  return float(ssp.n_wave) * ssp.locate_inv_h / float(ssp.n_locate) * span / float(nt - 1);
+}
+
+// Adjoint by star_bwd_dense_kernel: from the density at which 64 bins and the
+// margins no longer fit star_bwd_reg_kernel's 64 knots (0.95) to the one at which
+// they no longer fit the records (2.8).  Below, the registers win (0.67: 550 us
+// an adjoint call of 200 k stars to 1500 bins); above, every bin would be gathered
+// in either.
+static bool dense_knots(const rbx_ssp& ssp, const rbx_target& tg) {
+  if (!tg.ascending || ssp.locate_multi || tg.n < 2) return false;
+  const float knots = mean_knots(ssp, tg.n, tg.wmax - tg.wmin);
+  return knots >= 0.95f && knots <= 2.75f;
+}
+
 // Strided bins per lane of an axis of up to 4096 bins.  4, but where knots
 // are dense, the window of a wavefront's 256 bins does not fit its LDS (from 1.2
 // knots a bin: every bin searches memory) or takes long to stage, and 3 or 2
@@ -2285,7 +2453,7 @@ static bool sparse_knots(const rbx_ssp& ssp, const rbx_target& tg) {
 // 579 -> 538, 534, 617 with 3, 511, 543, 566 with 2.
 static int fused_bins(const rbx_ssp& ssp, int nt, float span) {
   if (ssp.locate_multi || nt < 2) return 4;
-  const float knots = float(ssp.n_wave) * ssp.locate_inv_h / float(ssp.n_locate) * span / float(nt - 1);
+  const float knots = mean_knots(ssp, nt, span);
   if (knots >= 1.15f && knots <= 2.9f && (nt <= 512 || (nt > 1536 && nt <= 2048))) return 2;
   if (knots >= 0.85f && (nt <= 768 || (nt > 1024 && nt <= 1536) || (nt > 2048 && nt <= 3072))) return 3;
   return 4;
@@ -2453,16 +2621,16 @@ int cube_bwd_impl(const rbx_ssp* ssp, const rbx_target* target, const rbx_stars*
   const SspView g = view_of(*ssp);
   const int32_t nt = target->n;
   // slabs of whole 64-bin groups, or of whole 256-bin blocks for the runs
-  const bool runs = sparse_knots(*ssp, *target);
+  const bool runs = sparse_knots(*ssp, *target), dense = dense_knots(*ssp, *target);
   const int unit = runs ? kBwdRunBins : kTile;
   const int slab_bins = ((nt + unit - 1) / unit + kBwdSlabs - 1) / kBwdSlabs * unit;
   const int64_t items = int64_t(kBwdSlabs) * ((n + t.waves - 1) / t.waves);
   const int64_t grid = item_grid(items, t.persist, 64 * t.waves);
   switch (t.waves) {
-    case 1: launch_bwd<1>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
-    case 2: launch_bwd<2>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
-    case 8: launch_bwd<8>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs); break;
-    default: launch_bwd<4>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs);
+    case 1: launch_bwd<1>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs, dense); break;
+    case 2: launch_bwd<2>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs, dense); break;
+    case 8: launch_bwd<8>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs, dense); break;
+    default: launch_bwd<4>(grid, s, g, *target, n, items, L.state, L.gradw, dcube, slab_bins, axav, L.vpart, L.apart, runs, dense);
   }
   if ((rc = check_launch(who))) return rc;
   hipLaunchKernelGGL(star_grad_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, g, *stars,
